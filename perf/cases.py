@@ -19,6 +19,9 @@ share the one HIP runtime of the process (torch is imported first), so
 
 Frames, pairs, contacts and hits are deterministic to the bit, which is the
 library's contract, so those cases compare exactly.
+
+All states work on one stream: the library's grid-synchronised kernels expect
+the device to run one stream's work at a time (see DYPHUR_COOP_LAUNCH).
 """
 import ctypes as C
 import math
@@ -59,10 +62,11 @@ def listed():
          "frames": 20},
         # Trajectory optimisation of thrown stacks: forward and backward, short horizon.
         {"name": "grad_stacks_256", "kind": "grad", "scene": "stack", "scenes": 256, "median": 64, "top": 64,
-         "substeps": 1, "frames": 20, "every": 10},
-        # The same over ragged mixed scenes with substeps (workgroup-sized scenes among them).
+         "substeps": 1, "at": 0, "frames": 20, "every": 10},
+        # The same over ragged mixed scenes with substeps (workgroup-sized scenes among them), a second into their
+        # run, when the lower bodies have landed.
         {"name": "grad_mixed_200", "kind": "grad", "scene": "mixed", "scenes": 200, "median": 128, "top": 600,
-         "substeps": 4, "frames": 10, "every": 5},
+         "substeps": 4, "at": 60, "frames": 10, "every": 5},
         # A lidar sweep over the 32 768-body pile.
         {"name": "rays_mixed_32768", "kind": "rays", "n": 32768, "at": 240, "rays": 65536},
         # Key sort of the compute layer: 63-bit keys with a payload, odd count.
@@ -89,7 +93,8 @@ def draw(rng):
         return {"kind": "grad", "scene": what, "scenes": _log(rng, 8, 256 if what == "stack" else 160),
                 "median": 64 if what == "stack" else rng.randrange(30, 150),
                 "top": 64 if what == "stack" else rng.randrange(200, 600),
-                "substeps": rng.choice([1, 2, 4]), "frames": rng.randrange(4, 12), "every": rng.choice([3, 5, 10])}
+                "substeps": rng.choice([1, 2, 4]), "at": rng.randrange(0, 60), "frames": rng.randrange(4, 12),
+                "every": rng.choice([3, 5, 10])}
     if kind == "rays":
         return {"kind": "rays", "n": _log(rng, 100, 40000), "at": rng.randrange(0, 200), "rays": _log(rng, 500, 200000)}
     return {"kind": "sort", "n": _log(rng, 1000, 3000000)}
@@ -194,6 +199,16 @@ def _piles(counts, rng):
 # ---------------------------------------------------------------------------
 # State in tensors
 # ---------------------------------------------------------------------------
+_streams = []
+
+
+def _stream():
+    """The program's one stream."""
+    if not _streams:
+        _streams.append(capi.Stream())
+    return _streams[0]
+
+
 class TensorBodies:
     """Body arrays as rows of one tensor, in capi.BodyView's layout."""
 
@@ -247,7 +262,7 @@ def _world(case, seed):
         sc = scenes.joint_chains(max(1, n // links), links, seed=seed)
     else:
         sc = _random_mixed(n, rng)
-    w = capi.World(sc)
+    w = capi.World(sc, _stream())
     w.bodies = TensorBodies(sc)
     torch.cuda.synchronize()
     for _ in range(case["at"]):
@@ -287,25 +302,24 @@ def prepare(case, seed):
         n = case["n"]
         keys = torch.from_numpy(rng.integers(0, 1 << 63, n, dtype=np.int64)).cuda()
         vals = torch.arange(n, dtype=torch.int32, device="cuda")
-        return {"kind": kind, "s": capi.Stream(), "from": (keys, vals), "to": (keys.clone(), vals.clone())}
+        return {"kind": kind, "s": _stream(), "from": (keys, vals), "to": (keys.clone(), vals.clone())}
     rng = np.random.default_rng(seed)
     if kind == "batch":
-        b = capi.Batch(_piles(_counts(case["scenes"], case["median"], 8, case["top"]), rng))
+        b = capi.Batch(_piles(_counts(case["scenes"], case["median"], 8, case["top"]), rng), _stream())
     elif case["scene"] == "stack":
         g = scenes.Pcg32(seed)
-        b = capi.Batch([scenes.diff_stack(g) for _ in range(case["scenes"])])
+        b = capi.Batch([scenes.diff_stack(g) for _ in range(case["scenes"])], _stream())
     else:
         b = capi.Batch([_random_mixed(int(c), rng, 0.5) for c in
-                        _counts(case["scenes"], case["median"], 16, case["top"])])
+                        _counts(case["scenes"], case["median"], 16, case["top"])], _stream())
     b.bodies = TensorBodies(b.merged)
     torch.cuda.synchronize()
-    if kind == "batch":
-        if case["at"]:
-            b.step(case["at"])
-        b.s.wait()
-        b.bodies.snapshot()
-        return {"kind": kind, "batch": b, "frames": case["frames"]}
+    if case["at"]:
+        b.step(case["at"], n_substeps=case.get("substeps", 1))
+    b.s.wait()
     b.bodies.snapshot()
+    if kind == "batch":
+        return {"kind": kind, "batch": b, "frames": case["frames"]}
     d = capi.Diff(b, case["frames"], case["every"], n_substeps=case["substeps"], tape_contacts_per_body=6.0)
     n = b.n_bodies
     # d/dx of a squared distance to targets about half a metre away, and a small weight on the velocities
