@@ -101,14 +101,6 @@ size_t scan_tmp_words(size_t n);
 int scan_exclusive(hipStream_t s, const uint32_t *in, uint32_t *out, size_t n, uint32_t *d_total,
                    uint32_t *tmp);
 
-// Stable LSD radix sort in one workgroup of (key, value) pairs over key bits
-// [begin_bit, end_bit).  Keys/values in (k0, v0); (k1, v1) are scratch of the
-// same size.  The result ends in (k0, v0).  vals may be null for key-only sorts.
-int radix_sort_u32(hipStream_t s, uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, size_t n,
-                   int begin_bit, int end_bit);
-int radix_sort_u64(hipStream_t s, uint64_t *k0, uint32_t *v0, uint64_t *k1, uint32_t *v1, size_t n,
-                   int begin_bit, int end_bit);
-
 // Block-wide helpers ----------------------------------------------------------
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 
