@@ -53,6 +53,9 @@ constexpr uint32_t kLdsClasses = 2048;  // block-aggregated class counting limit
 constexpr uint32_t kNone = 0xffffffffu;
 constexpr uint32_t kMaxColours = 64;
 constexpr uint32_t kMaxGridBlocks = 1024;  // grid-stride kernels over capacity-sized ranges
+// Bodies up to which assign_flow runs on one XCD (one XCD against the chip, mid-run piles: 2 000 bodies 38 against
+// 58 us, 5 000 54 / 81, 8 000 65 / 90, 12 000 80 / 101, 20 000 89 / 89, 32 768 250 / 98).
+constexpr uint32_t kAssignOneXcd = 16384;
 constexpr uint32_t kSweepXcc = 0;         // the XCD whose workgroups run the assignment and the sweep
 
 // Solver metadata (device words).  solve_prep zeroes all but kMErr, which
@@ -72,18 +75,15 @@ enum : uint32_t {
     kMNj = 12,           // joints solved
     kMJBad = 13,         // a joint of this solve failed validation
     kMLive = 14,         // a contact left live by its first iteration (sweep_flow)
-    kMBarAssign = 16,    // 2 words: grid barrier of assign_lists
+    kMBarAssign = 16,    // 2 words: grid barrier of assign_flow
     kMBarSweep = 18,     // 2 words: grid barrier of the sweeps (sweep_flow: after iteration 0)
     kMFcnt = 20,         // 3 words: frontier sizes
     kMRegSweep = 24,     // 2 words: check-in of sweep_xcd (participants, arrivals)
-    kMRegAssign = 26,    // 2 words: check-in of assign_lists
+    kMFree = 26,         // constraints between two static bodies
     kMRegMotor = 28,     // 2 words: check-in of joint_motors_xcd
     kMBarMotor = 30,     // 2 words: barrier of joint_motors_xcd
-    kMDeep = 32,         // a contact's chain is longer than 256 rounds (colour_flow)
-    kMQHead = 64,        // colour_flow's ready queue, one 128-byte line per counter:
-    kMQTail = 96,        //   positions claimed, entries pushed (after the first
-    kMQDone = 128,       //   frontier), contacts coloured
-    kMWords = 160,
+    kMRegAssign = 32,    // 2 words: check-in of assign_flow on one XCD
+    kMWords = 34,
 };
 constexpr uint32_t kErrBarrier = 2u, kErrCapacity = 4u, kErrAssign = 8u, kErrFlow = 16u, kErrJoint = 32u;
 
@@ -91,6 +91,15 @@ __device__ __forceinline__ uint32_t cls_of(uint64_t s) { return static_cast<uint
 
 __device__ __forceinline__ uint32_t grid_stride() { return gridDim.x * blockDim.x; }
 __device__ __forceinline__ uint32_t grid_tid() { return blockIdx.x * blockDim.x + threadIdx.x; }
+
+// What one end's body hands to the other in assign_flow, 16 bytes: the colours
+// used on it (its level on the reference-order path) and its round.  Bit 0 of
+// the first half and `round` of the second are non-zero once written, so each
+// half tells by itself whether it is there.
+struct alignas(16) FlowWord {
+    uint64_t lo;  // used << 1 | 1
+    uint64_t hi;  // (round + 1) << 1 | used >> 63
+};
 
 // Zeroes the per-solve state and publishes the constraint counts and the
 // path: the reference runs its constraints serially at <= 256 constraints
@@ -112,22 +121,31 @@ __device__ __forceinline__ void gather_body(const dy_body_view &bv, uint32_t i, 
 __global__ void solve_prep(dy_body_view bv, const uint32_t *__restrict__ ncp, uint32_t cap, uint32_t nj,
                            int force_serial, uint32_t *__restrict__ deg, uint32_t *__restrict__ fill,
                            uint64_t *__restrict__ used, uint32_t *__restrict__ ver, float *__restrict__ lam,
-                           uint32_t *__restrict__ hist, uint32_t *__restrict__ meta, float4 *__restrict__ dyn,
+                           FlowWord *__restrict__ flow, uint32_t *__restrict__ hist, uint32_t *__restrict__ meta,
+                           float4 *__restrict__ dyn,
                            float4 *__restrict__ sta) {
     const uint32_t nb = bv.n;
     const uint32_t n_raw = *ncp;
     const uint32_t nc = n_raw < cap ? n_raw : cap;
     const uint32_t ncon = nc + nj;
     const uint32_t top = nb > ncon ? nb : ncon;
+    const bool serial = force_serial || ncon <= 256u;
+    // dependency levels that the reference order may count (a rejected joint set can leave <= 256 contacts)
+    const uint32_t levels = serial || ncon < 256u ? ncon : 256u;
     for (uint32_t i = grid_tid(); i < top; i += grid_stride()) {
         if (i < nb) {
             deg[i] = 0;
             fill[i] = 0;
             used[i] = 0;
+            used[nb + i] = 0;
             ver[i] = 0;
             gather_body(bv, i, dyn, sta);
         }
-        if (i < ncon) lam[i] = 0.f;
+        if (i < ncon) {
+            lam[i] = 0.f;
+            flow[2u * i] = flow[2u * i + 1u] = FlowWord{0ull, 0ull};
+        }
+        if (i < levels) hist[i] = 0u;
     }
     const uint32_t i = grid_tid();
     if (i <= kMaxColours) hist[i] = 0;
@@ -136,7 +154,7 @@ __global__ void solve_prep(dy_body_view bv, const uint32_t *__restrict__ ncp, ui
         if (i == kMNc) v = ncon;
         if (i == kMNcc) v = nc;
         if (i == kMNj) v = nj;
-        if (i == kMSerial) v = (force_serial || ncon <= 256u) ? 1u : 0u;
+        if (i == kMSerial) v = serial ? 1u : 0u;
         meta[i] = v;
     }
     if (i == 0 && n_raw > cap) atomicOr(&meta[kMErr], kErrCapacity);
@@ -244,9 +262,10 @@ __global__ void solve_degree(Cons cs, const uint32_t *__restrict__ meta, const f
 }
 
 // Unordered per-body lists of dynamic endpoints: adj = (c << 1 | end), own = body.
-__global__ void solve_fill(Cons cs, const uint32_t *__restrict__ meta, const float *__restrict__ im,
+// Constraints between two static bodies get class 0 and round 1 here.
+__global__ void solve_fill(Cons cs, uint32_t *__restrict__ meta, const float *__restrict__ im,
                            const uint32_t *__restrict__ off, uint32_t *__restrict__ fill, uint32_t *__restrict__ adj,
-                           uint32_t *__restrict__ own) {
+                           uint32_t *__restrict__ own, uint32_t *__restrict__ cstat, uint64_t *__restrict__ state) {
     const uint32_t nc = meta[kMNc], ncc = meta[kMNcc];
     for (uint32_t c0 = grid_tid() & ~63u; c0 < nc; c0 += grid_stride()) {
         const uint32_t c = c0 + lane_id();
@@ -269,6 +288,13 @@ __global__ void solve_fill(Cons cs, const uint32_t *__restrict__ meta, const flo
             const uint32_t p = off[b] + atomicAdd(&fill[b], 1u);
             adj[p] = (c << 1) | 1u;
             own[p] = b;
+        }
+        if (c < nc) {
+            cstat[c] = (a == kNone || b == kNone) ? 1u : 0u;
+            if (a == kNone && b == kNone) {
+                state[c] = 1ull << 32;
+                atomicAdd(&meta[kMFree], 1u);
+            }
         }
     }
 }
@@ -344,12 +370,13 @@ __device__ __forceinline__ void block_append(bool pred, uint32_t val, uint32_t *
 
 // Per-body contact lists.  Every dynamic endpoint (contact c, end e) has an
 // entry adj[p] = (c << 1 | e) in its body's segment [off[x], off[x] + deg[x]),
-// and own[p] = x.  rank_entry places c at its rank in the body's order
-// (slot[off[x] + rank]) and records the rank per endpoint (crank[2c + e]).
+// and own[p] = x.  rank_entry places c at its rank in the body's order:
+// slot[off[x] + rank] = (c << 1 | e, 1 when the other end is static), and
+// records the rank per endpoint (crank[2c + e], for the rounds; may be null).
 // Cost per entry: one pass over the body's segment (L2-resident).
 __device__ __forceinline__ void rank_entry(uint32_t p, const uint32_t *__restrict__ adj,
                                            const uint32_t *__restrict__ own, const uint32_t *__restrict__ off,
-                                           const uint32_t *__restrict__ deg, int serial, uint32_t *__restrict__ slot,
+                                           const uint32_t *__restrict__ deg, const uint32_t *__restrict__ cstat, int serial, uint2 *__restrict__ slot,
                                            uint32_t *__restrict__ crank) {
     const uint32_t v = adj[p], x = own[p];
     const uint32_t c = v >> 1;
@@ -368,8 +395,8 @@ __device__ __forceinline__ void rank_entry(uint32_t p, const uint32_t *__restric
             rank += (q < n && (kq > kc || (kq == kc && q < self))) ? 1u : 0u;  // ties (a == b) by position
         }
     }
-    slot[beg + rank] = c;
-    crank[2u * c + (v & 1u)] = rank;
+    slot[beg + rank] = make_uint2(v, cstat[c]);
+    if (crank) crank[2u * c + (v & 1u)] = rank;
 }
 
 // Links contact c to its successor in both endpoint lists and counts the
@@ -378,7 +405,7 @@ __device__ __forceinline__ void rank_entry(uint32_t p, const uint32_t *__restric
 // endpoints are "none".
 __device__ __forceinline__ bool link_contact(uint32_t c, const Cons &cs, uint32_t ncc, const float *__restrict__ im,
                                              const uint32_t *__restrict__ off, const uint32_t *__restrict__ deg,
-                                             const uint32_t *__restrict__ slot, const uint32_t *__restrict__ crank,
+                                             const uint2 *__restrict__ slot, const uint32_t *__restrict__ crank,
                                              uint4 *__restrict__ lrec, uint32_t *__restrict__ pending) {
     uint32_t ends[2];
     cons_ends(cs, c, ncc, ends[0], ends[1]);
@@ -392,7 +419,7 @@ __device__ __forceinline__ bool link_contact(uint32_t c, const Cons &cs, uint32_
             continue;
         }
         const uint32_t r = crank[2u * c + e];
-        if (r + 1u < deg[x]) next[e] = slot[off[x] + r + 1u];
+        if (r + 1u < deg[x]) next[e] = slot[off[x] + r + 1u].x >> 1;
         wait += r != 0u ? 1u : 0u;
     }
     lrec[c] = make_uint4(ends[0], ends[1], next[0], next[1]);
@@ -405,29 +432,28 @@ __global__ __launch_bounds__(kSolveThreads) void list_rank(const uint32_t *__res
                                                            const uint32_t *__restrict__ off,
                                                            const uint32_t *__restrict__ deg,
                                                            const uint32_t *__restrict__ meta,
-                                                           uint32_t *__restrict__ slot, uint32_t *__restrict__ crank) {
+                                                           const uint32_t *__restrict__ cstat,
+                                                           uint2 *__restrict__ slot, uint32_t *__restrict__ crank) {
     const uint32_t total = meta[kMDyn];
     const int serial = static_cast<int>(meta[kMSerial]);
-    for (uint32_t p = grid_tid(); p < total; p += grid_stride()) rank_entry(p, adj, own, off, deg, serial, slot, crank);
+    for (uint32_t p = grid_tid(); p < total; p += grid_stride())
+        rank_entry(p, adj, own, off, deg, cstat, serial, slot, crank);
 }
 
 // Contacts heading every list of a dynamic endpoint form the first frontier
-// (fr0, size in fcnt[0]); the dataflow colouring's queue (queue[0, nc)) is
-// cleared to all ones.
+// (size in fcnt[0]) of the launch-per-round assignment.
 __global__ __launch_bounds__(kSolveThreads) void list_link(Cons cs, const uint32_t *__restrict__ meta,
                                                            const float *__restrict__ im,
                                                            const uint32_t *__restrict__ off,
                                                            const uint32_t *__restrict__ deg,
-                                                           const uint32_t *__restrict__ slot,
+                                                           const uint2 *__restrict__ slot,
                                                            const uint32_t *__restrict__ crank,
                                                            uint4 *__restrict__ lrec, uint32_t *__restrict__ pending,
-                                                           uint32_t *__restrict__ frontier, uint32_t *fcount,
-                                                           uint64_t *__restrict__ queue) {
+                                                           uint32_t *__restrict__ frontier, uint32_t *fcount) {
     const uint32_t nc = meta[kMNc], ncc = meta[kMNcc];
     for (uint32_t c0 = blockIdx.x * kSolveThreads; c0 < nc; c0 += gridDim.x * kSolveThreads) {
         const uint32_t c = c0 + threadIdx.x;
         const bool head = c < nc && link_contact(c, cs, ncc, im, off, deg, slot, crank, lrec, pending);
-        if (c < nc) queue[c] = ~0ull;
         block_append(head, c, frontier, fcount);
     }
 }
@@ -467,323 +493,346 @@ __device__ __forceinline__ uint32_t assign_one(uint32_t c, uint32_t round, int s
     return cls;
 }
 
-// Buffers of the cooperative class assignment.
+// Buffers of the class assignment.
 struct AssignBufs {
-    Cons cons;
-    const float *im;
-    const uint32_t *adj, *own, *off, *deg;
-    uint32_t *slot, *crank;
-    uint4 *lrec;
-    uint64_t *fq;  // colour_flow's queue: (round << 32) | contact
-    uint32_t *pending;
-    uint64_t *used, *state;
-    uint32_t *fr0, *fr1;
+    const uint32_t *adj, *own, *off, *deg, *cstat;
+    uint2 *slot;
+    FlowWord *flow;
+    uint64_t *body;  // 2 words a body: state of the bodies of threads that own several
+    uint64_t *state;
     uint32_t *meta, *hist, *boff, *bfill;
     uint32_t nbody;
 };
 
-// Touches every 128-byte line of [p, p + bytes) once across the participants
-// (gtid of gstride), so that the XCD's L2 holds the lines before the
-// dependent accesses of colour_flow reach them.
-__device__ __forceinline__ void touch_lines(const void *p, size_t bytes, uint32_t gtid, uint32_t gstride) {
-    const uint8_t *b = static_cast<const uint8_t *>(p);
-    for (size_t o = static_cast<size_t>(gtid) * 128u; o < bytes; o += static_cast<size_t>(gstride) * 128u) {
-        const uint32_t v = *reinterpret_cast<const uint32_t *>(b + o);
-        asm volatile("" ::"v"(v));
-    }
-}
-
-// Dataflow colouring: the JP assignment without round barriers.  A contact
-// can be coloured once the contacts ahead of it on both its lists are: then
-// used[a] | used[b] holds exactly its higher-priority neighbours' colours, as
-// in its JP round, and its round (the longest decreasing-priority chain
-// ending at it) is one more than the larger of its list predecessors'
-// rounds.  A predecessor decrements a successor's pending count and adds its
-// own round above bit 8 in the same atomic, so the last of a contact's (at
-// most two) predecessors learns the other's round from the returned value.
-// That lane continues with the successor itself (its list record loaded
-// while the predecessor was coloured); a second ready successor is pushed to
-// a queue (positions fr0[0, n0) hold the first frontier, then queue[0, ..)
-// entries (round << 32 | contact) in push order), from which lanes with
-// nothing in hand claim positions, one atomic per wave.  A claimed position
-// is read until its entry appears; it may never appear once every contact
-// is coloured, which ends the pass.  Writers wait for their stores (masks,
-// state) before the decrements; data written during the kernel is read with
-// agent-scope loads (the one-XCD handoff of assign_lists' rounds).
-// Progress: a claimed position below the queue's fill level is always
-// filled, so while uncoloured contacts remain some lane holds a ready one.
-// False on a timeout (kErrFlow).
-__device__ bool colour_flow(const AssignBufs &B, uint32_t nc, uint32_t *lhist, uint32_t &my_max,
-                            uint32_t &my_done, uint32_t &my_round) {
-    uint32_t *meta = B.meta;
-    uint64_t *queue = B.fq;
-    const uint32_t lane = lane_id();
-    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    const uint32_t n0 = ld_agent(&meta[kMFcnt]);
-    uint32_t cur = kNone, pos = kNone, round = 0, spins = 0, unpublished = 0;
-    uint4 rec = make_uint4(kNone, kNone, kNone, kNone);
-    bool have_rec = false;
-    for (;;) {
-        // lanes with nothing in hand claim queue positions
-        const bool need = cur == kNone && pos == kNone;
-        const uint64_t nm = __ballot(need);
-        if (nm) {
-            const uint32_t lead = static_cast<uint32_t>(__builtin_ctzll(nm));
-            uint32_t base = 0;
-            if (lane == lead) base = atomicAdd(&meta[kMQHead], static_cast<uint32_t>(__popcll(nm)));
-            base = __shfl(base, static_cast<int>(lead), 64);
-            if (need) pos = base + static_cast<uint32_t>(__popcll(nm & lt));
-        }
-        if (pos < nc) {
-            if (pos < n0) {
-                cur = B.fr0[pos];
-                round = 1u;
-                pos = kNone;
-                have_rec = false;
-            } else {
-                const uint64_t w = ld_agent(&queue[pos - n0]);
-                if (w != ~0ull) {
-                    cur = static_cast<uint32_t>(w);
-                    round = static_cast<uint32_t>(w >> 32);
-                    pos = kNone;
-                    have_rec = false;
+// Barrier among the first n workgroups of the launch, as grid_barrier.  With
+// `fence`, data stored before it by plain stores is seen by plain loads after
+// it; without, only what agent-scope atomics wrote.
+__device__ __forceinline__ void part_barrier(uint32_t *bar, uint32_t &gen, uint32_t n, uint32_t *err, bool fence) {
+    wait_vmem();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (fence) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        if (__hip_atomic_fetch_add(&bar[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1u) {
+            __hip_atomic_store(&bar[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            wait_vmem();
+            __hip_atomic_store(&bar[1], gen + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+            uint32_t spins = 0;
+            while (ld_agent(&bar[1]) == gen) {
+                __builtin_amdgcn_s_sleep(1);
+                if (++spins > kGridSpinLimit) {
+                    atomicOr(err, kErrBarrier);
+                    break;
                 }
             }
         }
-        // colour the contacts in hand
-        bool push = false;
-        uint64_t pushed = 0;
-        const bool work = cur != kNone;
-        if (work) {
-            if (!have_rec) rec = B.lrec[cur];
-            const uint64_t ua = rec.x != kNone ? ld_agent(&B.used[rec.x]) : 0ull;
-            const uint64_t ub = rec.y != kNone ? ld_agent(&B.used[rec.y]) : 0ull;
-            const uint4 none4 = make_uint4(kNone, kNone, kNone, kNone);
-            const uint4 rec_a = rec.z != kNone ? B.lrec[rec.z] : none4;  // the successors' records
-            const uint4 rec_b = rec.w != kNone ? B.lrec[rec.w] : none4;
-            const uint64_t u = ua | ub;
-            uint32_t cls;
-            if (u == ~0ull) {
-                atomicOr(&meta[kMOverflow], 1u);
-                cls = kMaxColours;
-            } else {
-                cls = static_cast<uint32_t>(__builtin_ctzll(~u));
-            }
-            const uint64_t bit = 1ull << (cls & 63u);
-            if (rec.x != kNone) B.used[rec.x] = ua | bit;
-            if (rec.y != kNone) B.used[rec.y] = ub | bit;
-            B.state[cur] = (static_cast<uint64_t>(round) << 32) | cls;
-            if (round > 256u) atomicOr(&meta[kMDeep], 1u);
-            wait_vmem();  // masks and state in the L2 before a successor can start
-            const uint32_t rr = round < 0xffffu ? round : 0xffffu;  // rounds past 256 only flag
-            const uint32_t add = (rr << 8) - 1u;
-            const uint32_t oa = rec.z != kNone ? atomicAdd(&B.pending[rec.z], add) : 0u;
-            const uint32_t ob = rec.w != kNone ? atomicAdd(&B.pending[rec.w], add) : 0u;
-            const bool ra = rec.z != kNone && (oa & 0xffu) == 1u, rb = rec.w != kNone && (ob & 0xffu) == 1u;
-            const uint32_t na = 1u + (rr > (oa >> 8) ? rr : (oa >> 8));
-            const uint32_t nb = 1u + (rr > (ob >> 8) ? rr : (ob >> 8));
-            my_max = cls > my_max ? cls : my_max;
-            my_round = round > my_round ? round : my_round;
-            ++my_done;
-            atomicAdd(&lhist[cls < kMaxColours ? cls : kMaxColours], 1u);
-            const uint32_t succ_b = rec.w;
-            if (ra) {
-                cur = rec.z;
-                rec = rec_a;
-                round = na;
-                have_rec = true;
-                push = rb;
-                pushed = (static_cast<uint64_t>(nb) << 32) | succ_b;
-            } else if (rb) {
-                cur = succ_b;
-                rec = rec_b;
-                round = nb;
-                have_rec = true;
-            } else {
-                cur = kNone;
-                have_rec = false;
-            }
-        }
-        // a second ready successor goes to the queue
-        const uint64_t pm = __ballot(push);
-        if (pm) {
-            const uint32_t lead = static_cast<uint32_t>(__builtin_ctzll(pm));
-            uint32_t base = 0;
-            if (lane == lead) base = atomicAdd(&meta[kMQTail], static_cast<uint32_t>(__popcll(pm)));
-            base = __shfl(base, static_cast<int>(lead), 64);
-            if (push) queue[base + static_cast<uint32_t>(__popcll(pm & lt))] = pushed;
-        }
-        unpublished += static_cast<uint32_t>(__popcll(__ballot(work)));
-        if (!__ballot(cur != kNone)) {
-            // the count is read only by idle waves: a wave adds its coloured
-            // contacts when it runs out of work
-            if (unpublished) {
-                if (lane == 0) atomicAdd(&meta[kMQDone], unpublished);
-                unpublished = 0;
-            }
-            if (ld_agent(&meta[kMQDone]) >= nc) return true;
-            __builtin_amdgcn_s_sleep(1);
-            if (++spins > kGridSpinLimit) {
-                if (lane == 0) atomicOr(&meta[kMErr], kErrFlow);
-                return false;
-            }
-            if ((spins & 255u) == 0u && (ld_agent(&meta[kMErr]) & kErrFlow)) return false;
-        }
+        if (fence) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    gen += 1u;
+    __syncthreads();
+}
+
+// Agent-scope access to a flow word: one 16-byte access, each half of it a
+// single-copy 64-bit one (readers check both halves).
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ FlowWord flow_word(const u32x4 &v) {
+    return FlowWord{v.x | static_cast<uint64_t>(v.y) << 32, v.z | static_cast<uint64_t>(v.w) << 32};
+}
+// On one XCD the word only has to reach its L2; readers skip the L1.  A store
+// of more than 8 bytes reads its data one wait state after issue.
+template <bool ONE_XCD>
+__device__ __forceinline__ void st_flow(FlowWord *p, uint64_t used, uint32_t round) {
+    const u32x4 v = {static_cast<uint32_t>(used << 1) | 1u, static_cast<uint32_t>(used >> 31),
+                     ((round + 1u) << 1) | static_cast<uint32_t>(used >> 63), (round + 1u) >> 31};
+    if (ONE_XCD) asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+    else asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+}
+// Both words, the two loads in flight together.
+constexpr uint32_t kFlowAhead = 2;
+__device__ __forceinline__ void ld_flow(const FlowWord *const (&p)[kFlowAhead], FlowWord (&f)[kFlowAhead]) {
+    u32x4 v, w;
+    asm volatile("global_load_dwordx4 %0, %2, off sc1\n\tglobal_load_dwordx4 %1, %3, off sc1\n\ts_waitcnt vmcnt(0)"
+                 : "=&v"(v), "=&v"(w) : "v"(p[0]), "v"(p[1]) : "memory");
+    f[0] = flow_word(v);
+    f[1] = flow_word(w);
+}
+
+constexpr uint32_t kTold = 0x80000000u;  // in a stored `next`: the word of that entry is out
+
+// What a thread's (then a workgroup's) contacts add to the assignment's
+// statistics.
+struct AssignStats {
+    uint32_t max_cls, max_round, done;
+};
+
+// A body on its way through its ordered contact list, with the next entries.
+struct BodyFlow {
+    uint64_t used;   // colours used on it so far; reference order: its level
+    uint32_t round;  // round of its last contact
+    uint32_t next;   // entries done
+    uint32_t told;   // entries whose word is out: next or next + 1
+    uint32_t have;   // entries in e: next, next + 1, ..
+    uint2 e[kFlowAhead];
+};
+
+template <bool ONE_XCD>
+__device__ __forceinline__ void flow_tell(const AssignBufs &B, BodyFlow &F) {
+    if (F.have != 0u && F.told == F.next) {
+        F.told += 1u;
+        if (F.e[0].y == 0u) st_flow<ONE_XCD>(B.flow + F.e[0].x, F.used, F.round);
     }
 }
 
-// JP rounds over frontiers in one cooperative launch.  Round r assigns the
-// contacts that head the ordered lists of all their dynamic endpoints: on a
-// body's list every earlier contact is a higher-priority neighbour, so these
-// are exactly the contacts whose higher-priority neighbours were all assigned
-// before round r — the ones the reference colours in its round r.  A body
-// heads at most one contact per round, so the contact owns its bodies' masks
-// of used colours during the round.  Values written in a round are read only
-// after the barrier that ends it.  Frontier sizes rotate over fcnt[0..2]
-// (round r appends to fcnt[r % 3]).
+// Takes body state F (list entries slot[0, n)) as far as the other bodies'
+// words that are there allow, at most the entries in hand: true when it went
+// on.  The words of the entries ahead are read along with the next one's, so
+// that a run of contacts whose other bodies wait for this one costs one read.
+template <bool ONE_XCD>
+__device__ __forceinline__ bool flow_step(const AssignBufs &B, const uint2 *slot, uint32_t n, int serial, BodyFlow &F,
+                                          uint32_t *lhist, AssignStats &S) {
+    flow_tell<ONE_XCD>(B, F);
+    const FlowWord *p[kFlowAhead];
+    FlowWord o[kFlowAhead];
+#pragma unroll
+    for (uint32_t k = 0; k < kFlowAhead; ++k) p[k] = B.flow + (F.e[k].x ^ 1u);
+    const uint32_t at = F.next + F.have;
+    const uint2 in0 = at < n ? slot[at] : make_uint2(0u, 0u), in1 = at + 1u < n ? slot[at + 1u] : make_uint2(0u, 0u);
+    ld_flow(p, o);
+    uint32_t m = 0;
+    while (F.have != 0u && (F.e[0].y != 0u || (o[0].lo != 0ull && o[0].hi != 0ull))) {
+        const uint32_t c = F.e[0].x >> 1;
+        const bool alone = F.e[0].y != 0u;  // the other end is static
+        if (m != 0u && !alone) st_flow<ONE_XCD>(B.flow + F.e[0].x, F.used, F.round);
+        uint64_t used = F.used;
+        uint32_t round = F.round;
+        if (!alone) {
+            const uint64_t ou = (o[0].lo >> 1) | (o[0].hi << 63);
+            const uint32_t r = static_cast<uint32_t>(o[0].hi >> 1) - 1u;
+            used = serial ? (used > ou ? used : ou) : (used | ou);
+            round = round > r ? round : r;
+        }
+        round += 1u;
+        uint32_t cls;
+        if (serial) {
+            cls = static_cast<uint32_t>(used);
+            F.used = used + 1ull;
+        } else {
+            cls = kMaxColours;
+            if (used != ~0ull) cls = static_cast<uint32_t>(__builtin_ctzll(~used));
+            F.used |= 1ull << (cls & 63u);
+        }
+        F.round = round;
+        if (alone || (F.e[0].x & 1u) == 0u) {  // one of its bodies records the contact
+            B.state[c] = (static_cast<uint64_t>(round) << 32) | cls;
+            S.max_cls = cls > S.max_cls ? cls : S.max_cls;
+            S.max_round = round > S.max_round ? round : S.max_round;
+            S.done += 1u;
+            if (serial) atomicAdd(&B.hist[cls], 1u);
+            else atomicAdd(&lhist[cls], 1u);
+        }
+        m += 1u;
+        F.have -= 1u;
+#pragma unroll
+        for (uint32_t k = 0; k + 1u < kFlowAhead; ++k) {
+            F.e[k] = F.e[k + 1u];
+            o[k] = o[k + 1u];
+        }
+    }
+    F.next += m;
+    if (m) F.told = F.next;
+    // up to two new entries come in; a window with room for one takes the first
+    const uint32_t add = at + 1u < n ? 2u : (at < n ? 1u : 0u);
+#pragma unroll
+    for (uint32_t k = 0; k < kFlowAhead; ++k) {
+        if (k == F.have) F.e[k] = in0;
+        if (k == F.have + 1u) F.e[k] = in1;
+    }
+    F.have += add;
+    if (F.have > kFlowAhead) F.have = kFlowAhead;
+    return m != 0u;
+}
+
+// Takes the bodies gtid, gtid + stride, ... through their lists.  Progress:
+// the lists follow one total order of the contacts, so the first contact not
+// done heads both its bodies' lists, and no thread waits for one body while
+// another of its own could go on.  False on a timeout (kErrFlow).
+template <bool ONE_XCD>
+__device__ __forceinline__ bool flow_bodies(const AssignBufs &B, int serial, uint32_t gtid, uint32_t stride,
+                                            uint32_t *lhist, AssignStats &S) {
+    const uint32_t nb = B.nbody;
+    const bool several = nb > stride;
+    uint32_t x = gtid, spins = 0, left = 0;
+    const uint2 *slot = B.slot;
+    uint32_t n = 0;
+    BodyFlow F{};
+    if (several) {
+        for (uint32_t y = gtid; y < nb; y += stride) left += B.deg[y] != 0u ? 1u : 0u;
+    } else if (x < nb) {
+        n = B.deg[x];
+        slot += B.off[x];
+        left = n ? 1u : 0u;
+    }
+    while (__ballot(left != 0u)) {
+        bool got = false;
+        if (several) {
+            if (left && x < nb) {
+                n = B.deg[x];
+                const uint64_t w1 = B.body[2u * static_cast<size_t>(x) + 1u];
+                F.used = B.body[2u * static_cast<size_t>(x)];
+                F.round = static_cast<uint32_t>(w1);
+                F.next = static_cast<uint32_t>(w1 >> 32) & ~kTold;
+                F.told = F.next + ((w1 >> 63) ? 1u : 0u);
+                F.have = 0u;
+                if (F.next < n) {
+                    slot = B.slot + B.off[x];
+                    (void)flow_step<ONE_XCD>(B, slot, n, serial, F, lhist, S);  // fetches the entries
+                    while (F.next < n && flow_step<ONE_XCD>(B, slot, n, serial, F, lhist, S)) got = true;
+                    if (F.next == n) left -= 1u;
+                    B.body[2u * static_cast<size_t>(x)] = F.used;
+                    B.body[2u * static_cast<size_t>(x) + 1u] =
+                        F.round | static_cast<uint64_t>(F.next | (F.told != F.next ? kTold : 0u)) << 32;
+                }
+            }
+            x += stride;
+            if (x - gtid >= nb) x = gtid;  // the same round of the range on every thread of a wave
+        } else if (left) {
+            got = flow_step<ONE_XCD>(B, slot, n, serial, F, lhist, S);
+            if (F.next == n) left = 0u;
+        }
+        if (__ballot(got)) {
+            spins = 0;
+            continue;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        if (++spins > kGridSpinLimit) {
+            if (lane_id() == 0) atomicOr(&B.meta[kMErr], kErrFlow);
+            return false;
+        }
+        if ((spins & 255u) == 0u && (ld_agent(&B.meta[kMErr]) & (kErrFlow | kErrBarrier))) return false;
+    }
+    return true;
+}
+// Class assignment of a solve in one launch, a thread per body.
 //
-// When the colouring overflows 64 colours or needs more than 256 rounds, the
-// lists are re-ranked in contact order and the rounds re-run as dependency
-// levels: the reference's run_serial order.  The kernel ends with the class
-// offsets (boff[0..k]), zeroed per-class fill counters and the statistics.
-// Like the sweep, it runs on the workgroups of one XCD (see xcd_barrier):
-// frontier entries, used-colour masks and counters written during the kernel
-// are read at agent scope (L2), pending counts are L2 atomics.
-__global__ __launch_bounds__(1024) void assign_lists(AssignBufs B) {
+// Coloured path: a contact's higher-priority neighbours are the contacts ahead
+// of it on its bodies' lists, so its colour is the lowest one used by neither
+// body when it heads both lists, and its JP round (the longest
+// decreasing-priority chain ending at it) one more than the larger of the
+// bodies' rounds.  A thread takes its body along the body's list: it writes
+// the body's colours and round to the contact's word of its end, waits for the
+// other body's word, and both threads work out the same class.  When the
+// colouring overflows 64 colours or needs more than 256 rounds, the lists are
+// ranked again in contact order and the same flow gives dependency levels: the
+// reference's run_serial order, which is also the order from the start at
+// <= 256 contacts.
+//
+// Bound by the chain of rounds (35 on a settled stack of 1 024 boxes, 65 on a
+// settled pile of 32 768 bodies): a step of it is one store and one load, with
+// no atomic, queue or acknowledged store, and the words of two entries are
+// read at a time.  A word carries all that is handed over, so any of the chip's
+// workgroups may take part: a step is then about 1.5 us, from beyond the L2s,
+// but the waiting threads' loads spread over the chip.  On the workgroups of
+// one XCD (ONE_XCD) it goes through that XCD's L2, which is faster until the
+// loads of the waiting threads fill it: 5 000 bodies 57 against 79 us, 32 768
+// 250 against 98 us.  Against a queue of ready contacts served by one XCD with
+// an atomic per hand-over: 1 024 boxes 78 -> 47 us, 5 000 bodies 128 -> 57,
+// 32 768 186 -> 98, 98 305 425 -> 170 (and no kernel that links the lists).
+//
+// The kernel ends with the class offsets (boff[0..k]), zeroed per-class fill
+// counters and the statistics.
+template <bool ONE_XCD>
+__global__ __launch_bounds__(1024) void assign_flow(AssignBufs B) {
     __shared__ uint32_t lhist[kMaxColours + 1];
+    __shared__ uint32_t s_stat[3];
+    __shared__ uint32_t s_scan[17];
     uint32_t *meta = B.meta;
-    uint32_t *bar = meta + kMBarAssign, *fcnt = meta + kMFcnt, *err = meta + kMErr;
-    uint32_t bidx = 0, nblk = 0;
-    if (!xcd_checkin(kSweepXcc, meta + kMRegAssign, err, kErrBarrier, bidx, nblk)) return;
-    uint32_t gen = 0;
-    const uint32_t gtid = bidx * blockDim.x + threadIdx.x, gstride = nblk * blockDim.x;
-    const uint32_t lane = lane_id(), wave0 = gtid & ~63u;
+    uint32_t *bar = meta + kMBarAssign, *err = meta + kMErr;
+    uint32_t bidx = blockIdx.x, nblk = gridDim.x;
+    if (ONE_XCD && !xcd_checkin(kSweepXcc, meta + kMRegAssign, err, kErrBarrier, bidx, nblk)) return;
+    const uint32_t nt = blockDim.x;
+    const uint32_t gtid = bidx * nt + threadIdx.x, stride = nblk * nt;
     const uint32_t nc = meta[kMNc];
+    uint32_t gen = 0;
     int serial = static_cast<int>(meta[kMSerial]);
-    uint32_t my_max = 0, my_done = 0, rounds = 0, running = 0;
-    bool exceeded = false;
     for (int pass = 0; pass < 2; ++pass) {
-        for (uint32_t k = threadIdx.x; k <= kMaxColours; k += blockDim.x) lhist[k] = 0;
+        for (uint32_t k = threadIdx.x; k <= kMaxColours; k += nt) lhist[k] = 0u;
+        if (threadIdx.x < 3u) s_stat[threadIdx.x] = 0u;
         __syncthreads();
-        my_max = 0;
-        my_done = 0;
-        running = 0;
-        exceeded = false;
-        const uint32_t max_rounds = serial ? nc + 1u : 256u;
-        uint32_t *cur = B.fr0, *nxt = B.fr1;
-        uint32_t ncur = ld_agent(&fcnt[0]), round = 1;
-        if (!serial) {  // the colouring as dataflow; rounds only for the reference order
-            touch_lines(B.used, sizeof(uint64_t) * B.nbody, gtid, gstride);
-            touch_lines(B.lrec, sizeof(uint4) * nc, gtid, gstride);
-            touch_lines(B.pending, sizeof(uint32_t) * nc, gtid, gstride);
-            touch_lines(B.fq, sizeof(uint64_t) * nc, gtid, gstride);
-            touch_lines(B.fr0, sizeof(uint32_t) * ld_agent(&fcnt[0]), gtid, gstride);
-            uint32_t my_round = 0;
-            (void)colour_flow(B, nc, lhist, my_max, my_done, my_round);
-            my_round = wave_max_u32(my_round);
-            if (lane == 0 && my_round) atomicMax(&meta[kMRounds], my_round);
-            ncur = 0;
-        }
-        for (; ncur > 0; ++round) {
-            if (round > max_rounds) {  // deeper than the reference allows (uniform)
-                exceeded = true;
-                break;
-            }
-            if (serial && gtid == 0) B.boff[round - 1] = running;  // class round-1 = this frontier
-            running += ncur;
-            uint32_t *nxt_count = &fcnt[round % 3];
-            if (gtid == 0) fcnt[(round + 1) % 3] = 0u;
-            for (uint32_t i0 = wave0; i0 < ncur; i0 += gstride) {
-                const uint32_t i = i0 + lane;
-                bool ready[2] = {false, false};
-                uint32_t nx[2] = {0u, 0u};
-                if (i < ncur) {
-                    const uint32_t cls = assign_one(ld_agent(&cur[i]), round, serial, B.lrec, B.pending, B.used,
-                                                    B.state, meta, ready, nx);
-                    my_max = cls > my_max ? cls : my_max;
-                    ++my_done;
-                    if (!serial) atomicAdd(&lhist[cls < kMaxColours ? cls : kMaxColours], 1u);
-                }
-                wave_append<2>(ready, nx, nxt, nxt_count);
-            }
-            xcd_barrier(bar, gen, nblk, err, kErrBarrier);
-            ncur = ld_agent(&fcnt[round % 3]);
-            uint32_t *t = cur; cur = nxt; nxt = t;
-        }
-        rounds = round - 1u;
-        xcd_barrier(bar, gen, nblk, err, kErrBarrier);  // overflow flags of the last round
-        if (!serial) {
-            rounds = ld_agent(&meta[kMRounds]);
-            exceeded = ld_agent(&meta[kMDeep]) != 0u;  // a timeout leaves contacts unassigned: kErrAssign
-        }
-        const bool fallback = !serial && (exceeded || ld_agent(&meta[kMOverflow]) != 0u);
-        if (!fallback) break;
-        // The reference's serial path: contact order, classes = dependency
-        // levels.  The lists are rebuilt here, so the barriers around the
-        // rebuild also make plain loads of them see the other workgroups'
-        // stores.
-        serial = 1;
+        AssignStats S{0u, 0u, 0u};
+        (void)flow_bodies<ONE_XCD>(B, serial, gtid, stride, lhist, S);  // a timeout leaves contacts unassigned: kErrAssign
         if (gtid == 0) {
+            // constraints between two static bodies are on no list: class 0, round 1 (solve_fill)
+            const uint32_t free_ones = meta[kMFree];
+            if (free_ones) {
+                S.done += free_ones;
+                S.max_round = S.max_round > 1u ? S.max_round : 1u;
+                atomicAdd(&B.hist[0], free_ones);
+            }
+        }
+        S.max_cls = wave_max_u32(S.max_cls);
+        S.max_round = wave_max_u32(S.max_round);
+        S.done = wave_sum_u32(S.done);
+        if (lane_id() == 0) {
+            atomicMax(&s_stat[0], S.max_cls);
+            atomicMax(&s_stat[1], S.max_round);
+            atomicAdd(&s_stat[2], S.done);
+        }
+        __syncthreads();
+        if (threadIdx.x == 0 && s_stat[2]) {
+            atomicMax(&meta[kMMaxCls], s_stat[0]);
+            atomicMax(&meta[kMRounds], s_stat[1]);
+            atomicAdd(&meta[kMAssigned], s_stat[2]);
+        }
+        if (!serial)
+            for (uint32_t k = threadIdx.x; k <= kMaxColours; k += nt)
+                if (lhist[k]) atomicAdd(&B.hist[k], lhist[k]);
+        part_barrier(bar, gen, nblk, err, false);
+        if (serial) break;
+        const uint32_t rounds = ld_agent(&meta[kMRounds]);
+        const bool overflow = ld_agent(&B.hist[kMaxColours]) != 0u;
+        if (rounds <= 256u && !overflow) break;
+        // The reference's serial path.
+        serial = 1;
+        part_barrier(bar, gen, nblk, err, false);  // every workgroup has read the statistics
+        if (gtid == 0) {
+            meta[kMOverflow] = overflow ? 1u : 0u;
             meta[kMSerial] = 1u;
-            meta[kMColourRounds] = exceeded ? 257u : rounds;
-            fcnt[0] = 0u;
-            fcnt[1] = 0u;
-            fcnt[2] = 0u;
+            meta[kMColourRounds] = rounds > 256u ? 257u : rounds;
+            meta[kMRounds] = 0u;
+            meta[kMMaxCls] = 0u;
+            meta[kMAssigned] = 0u;
         }
         const uint32_t total = meta[kMDyn];
-        for (uint32_t p = gtid; p < total; p += gstride)
-            rank_entry(p, B.adj, B.own, B.off, B.deg, 1, B.slot, B.crank);
-        xcd_barrier(bar, gen, nblk, err, kErrBarrier, true);
-        for (uint32_t c0 = wave0; c0 < nc; c0 += gstride) {
-            const uint32_t c = c0 + lane;
-            const bool pred[1] = {c < nc && link_contact(c, B.cons, meta[kMNcc], B.im, B.off, B.deg, B.slot,
-                                                         B.crank, B.lrec, B.pending)};
-            const uint32_t val[1] = {c};
-            wave_append<1>(pred, val, B.fr0, &fcnt[0]);
+        for (uint32_t p = gtid; p < total; p += stride)
+            rank_entry(p, B.adj, B.own, B.off, B.deg, B.cstat, 1, B.slot, nullptr);
+        for (uint32_t k = gtid; k < nc || k <= kMaxColours; k += stride) B.hist[k] = 0u;
+        for (uint32_t k = gtid; k < nc; k += stride) B.flow[2u * k] = B.flow[2u * k + 1u] = FlowWord{0ull, 0ull};
+        for (uint32_t k = gtid; k < B.nbody; k += stride)
+            B.body[2u * static_cast<size_t>(k)] = B.body[2u * static_cast<size_t>(k) + 1u] = 0ull;
+        part_barrier(bar, gen, nblk, err, true);
+    }
+    if (bidx != 0) return;
+    // Class offsets: exclusive scan of the class sizes.
+    const uint32_t rounds = ld_agent(&meta[kMRounds]);
+    const bool ok = ld_agent(&meta[kMAssigned]) == nc;
+    const uint32_t ncls = !ok || nc == 0u ? 0u : ld_agent(&meta[kMMaxCls]) + 1u;
+    uint32_t run = 0;
+    for (uint32_t k0 = 0; k0 < ncls; k0 += nt) {
+        const uint32_t k = k0 + threadIdx.x;
+        uint32_t total;
+        const uint32_t off = block_exclusive_scan(k < ncls ? ld_agent(&B.hist[k]) : 0u, s_scan, total);
+        if (k < ncls) {
+            B.boff[k] = run + off;
+            B.bfill[k] = 0u;
         }
-        xcd_barrier(bar, gen, nblk, err, kErrBarrier, true);
+        run += total;
     }
-    // Class sizes: per-block colour histograms, or the frontier sizes.
-    if (!serial) {
-        __syncthreads();
-        for (uint32_t k = threadIdx.x; k <= kMaxColours; k += blockDim.x)
-            if (lhist[k]) atomicAdd(&B.hist[k], lhist[k]);
-    }
-    my_max = wave_max_u32(my_max);
-    my_done = wave_sum_u32(my_done);
-    if (lane == 0 && my_done) {
-        atomicMax(&meta[kMMaxCls], my_max);
-        atomicAdd(&meta[kMAssigned], my_done);
-    }
-    xcd_barrier(bar, gen, nblk, err, kErrBarrier);
-    const bool ok = !exceeded && ld_agent(&meta[kMAssigned]) == nc;
-    uint32_t ncls = 0;
-    if (ok) ncls = serial ? rounds : (nc ? ld_agent(&meta[kMMaxCls]) + 1u : 0u);
-    if (gtid == 0) {
+    if (threadIdx.x == 0) {
         if (!ok) atomicOr(err, kErrAssign);
         meta[kMRounds] = rounds;
         meta[kMNcls] = ncls;
-        if (serial) B.boff[ncls] = ok ? running : 0u;
+        B.boff[ncls] = run;
     }
-    if (!serial && gtid < 64u) {
-        // class offsets: exclusive scan of the <= 65 class sizes by one wave
-        const uint32_t h0 = gtid < ncls ? ld_agent(&B.hist[gtid]) : 0u;
-        const uint32_t h1 = gtid + 64u < ncls ? ld_agent(&B.hist[gtid + 64u]) : 0u;
-        uint32_t s0 = h0, s1 = h1;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t t0 = __shfl_up(s0, d, 64), t1 = __shfl_up(s1, d, 64);
-            if (lane >= static_cast<uint32_t>(d)) {
-                s0 += t0;
-                s1 += t1;
-            }
-        }
-        const uint32_t tot0 = __shfl(s0, 63, 64), tot1 = __shfl(s1, 63, 64);
-        if (gtid < ncls) B.boff[gtid] = s0 - h0;
-        if (gtid + 64u < ncls) B.boff[gtid + 64u] = tot0 + s1 - h1;
-        if (gtid == 0) B.boff[ncls] = tot0 + tot1;
-    }
-    for (uint32_t k = gtid; k < ncls; k += gstride) B.bfill[k] = 0u;
 }
 
 // One round per launch (used when a cooperative launch is unavailable or
@@ -1515,14 +1564,14 @@ struct dy_xpbd_s {
     uint32_t cap = 0;
     float *lam = nullptr;
     uint64_t *state = nullptr;
-    uint32_t *adj = nullptr, *own = nullptr, *slot = nullptr, *crank = nullptr, *pending = nullptr;
+    uint32_t *adj = nullptr, *own = nullptr, *crank = nullptr, *cstat = nullptr, *pending = nullptr;
     uint32_t *fr0 = nullptr, *fr1 = nullptr;
     uint32_t *boff = nullptr, *bfill = nullptr, *hist = nullptr, *rec_id = nullptr, *cpos = nullptr;
-    uint32_t *meta = nullptr;  // kMWords device words, inside meta_block
-    uint8_t *meta_block = nullptr;
+    uint32_t *meta = nullptr;  // kMWords device words
     uint4 *lrec = nullptr, *rseq = nullptr;
     uint2 *rec_ab = nullptr;
-    uint64_t *fq = nullptr;
+    FlowWord *flow = nullptr;
+    uint2 *slot = nullptr;
     float4 *rec_p0 = nullptr, *rec_p1 = nullptr;
     DevBuf<uint32_t> deg, off, fill, scan_tmp, ver;
     DevBuf<uint64_t> used;
@@ -1578,6 +1627,7 @@ int sync_meta(dy_xpbd_s *x) {
     x->stats.rounds = m[kMRounds];
     x->stats.overflow = m[kMOverflow];
     x->stats.dyn_endpoints = m[kMDyn];
+
     if (m[kMErr] == kErrJoint) return DY_ERR_INVALID_ARG;
     return m[kMErr] ? DY_ERR_INTERNAL : DY_OK;
 }
@@ -1605,8 +1655,8 @@ int collect_timing(dy_xpbd_s *x) {
 // The constraint-indexed buffers, for c constraints (contacts + joints).
 void free_constraint_bufs(dy_xpbd_s *x) {
     void **ptrs[] = {(void **)&x->lam, (void **)&x->state, (void **)&x->adj, (void **)&x->own, (void **)&x->slot,
-                     (void **)&x->crank, (void **)&x->pending, (void **)&x->fr0, (void **)&x->fr1,
-                     (void **)&x->lrec, (void **)&x->fq, (void **)&x->boff, (void **)&x->bfill, (void **)&x->hist,
+                     (void **)&x->crank, (void **)&x->cstat, (void **)&x->pending, (void **)&x->fr0, (void **)&x->fr1,
+                     (void **)&x->lrec, (void **)&x->flow, (void **)&x->boff, (void **)&x->bfill, (void **)&x->hist,
                      (void **)&x->rec_id, (void **)&x->cpos, (void **)&x->rseq, (void **)&x->rec_ab,
                      (void **)&x->rec_p0, (void **)&x->rec_p1};
     for (void **p : ptrs)
@@ -1631,11 +1681,12 @@ hipError_t alloc_constraint_bufs(dy_xpbd_s *x, uint32_t n_con) {
     dalloc(x->own, 2 * c);
     dalloc(x->slot, 2 * c);
     dalloc(x->crank, 2 * c);
+    dalloc(x->cstat, c);
     dalloc(x->pending, c);
     dalloc(x->fr0, c);
     dalloc(x->fr1, c);
     dalloc(x->lrec, c);
-    dalloc(x->fq, c);
+    dalloc(x->flow, 2 * c);
     dalloc(x->boff, ncls);
     dalloc(x->bfill, ncls);
     dalloc(x->hist, ncls);
@@ -1672,58 +1723,11 @@ void xp_free(dy_xpbd_s *x) {
     if (x->ev_meta) (void)hipEventDestroy(x->ev_meta);
     if (x->h_meta) (void)hipHostFree(x->h_meta);
     free_constraint_bufs(x);
-    void *ptrs[] = {x->meta_block, x->jpk, x->jend};
+    void *ptrs[] = {x->meta, x->jpk, x->jend};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     x->deg.release(); x->off.release(); x->fill.release(); x->scan_tmp.release(); x->ver.release();
     x->used.release(); x->dyn.release(); x->sta.release();
-}
-
-// Placement of the metadata words.  Device atomics are served beyond the
-// XCD's L2 and their latency depends on the address: of two lines 8 KiB
-// apart, one is typically served about a third faster than the other from a
-// given XCD, and which one depends on the physical page.  The assignment's
-// queue counters (kMQHead, kMQTail, kMQDone) take an atomic per wave and
-// claim, so the metadata goes into whichever half of a 16 KiB block answers
-// faster from the assignment's XCD, measured once at creation by chains of
-// dependent atomics on each half's queue-counter line.
-constexpr uint32_t kMetaHalf = 8192u, kMetaBlock = 2u * kMetaHalf;
-constexpr uint32_t kMetaProbeChain = 64u;
-static_assert(kMWords * sizeof(uint32_t) <= kMetaHalf, "metadata fits half the block");
-
-__global__ void meta_place_probe(uint32_t *block, uint32_t *elect, uint64_t *ticks) {
-    if (threadIdx.x != 0 || xcc_id() != kSweepXcc) return;
-    if (atomicCAS(elect, 0u, 1u) != 0u) return;  // one workgroup on that XCD measures
-    for (uint32_t h = 0; h < 2u; ++h) {
-        uint32_t *p = block + h * (kMetaHalf / 4u) + kMQHead;
-        uint32_t v = 0;
-        const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-        for (uint32_t i = 0; i < kMetaProbeChain; ++i) v = atomicAdd(p + (v >> 31), 1u);  // v < 2^31: dependent chain
-        ticks[h] = __builtin_amdgcn_s_memrealtime() - t0 + (v >> 31);
-    }
-}
-
-// Chooses x->meta inside x->meta_block (allocated, kMetaBlock bytes) and
-// zeroes the block.  Synchronous (creation only).
-hipError_t place_meta(dy_xpbd_s *x, hipStream_t st) {
-    uint32_t *scratch = nullptr;  // [0] election, [2..5] two 64-bit tick counts
-    hipError_t e = hipMalloc(reinterpret_cast<void **>(&scratch), 8 * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMemsetAsync(x->meta_block, 0, kMetaBlock, st);
-    if (e == hipSuccess) e = hipMemsetAsync(scratch, 0, 8 * sizeof(uint32_t), st);
-    uint64_t ticks[2] = {0, 0};
-    if (e == hipSuccess) {
-        meta_place_probe<<<8, 64, 0, st>>>(reinterpret_cast<uint32_t *>(x->meta_block), scratch,
-                                            reinterpret_cast<uint64_t *>(scratch + 2));
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipMemcpyAsync(ticks, scratch + 2, sizeof(ticks), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (scratch) (void)hipFree(scratch);
-    // the second half only when it measured clearly faster (both zero: no measurement)
-    const bool second = ticks[0] > 0 && ticks[1] > 0 && ticks[1] * 10u < ticks[0] * 9u;
-    x->meta = reinterpret_cast<uint32_t *>(x->meta_block + (second ? kMetaHalf : 0u));
-    if (e == hipSuccess) e = hipMemsetAsync(x->meta_block, 0, kMetaBlock, st);
-    return e;
 }
 
 int env_int(const char *name, int dflt) {
@@ -1760,9 +1764,12 @@ int query_coop(dy_xpbd_s *x) {
     }
     if (!coop) return DY_OK;
     int per_cu = 0;
-    DY_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(assign_lists),
+    int per_cu_xcd = 0;
+    DY_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(assign_flow<false>),
                                                         x->assign_threads, 0));
-    x->coop_assign_max = per_cu * x->device_cus;
+    DY_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_xcd, reinterpret_cast<const void *>(assign_flow<true>),
+                                                        x->assign_threads, 0));
+    x->coop_assign_max = (per_cu < per_cu_xcd ? per_cu : per_cu_xcd) * x->device_cus;
     const void *fns[4][2] = {
         {reinterpret_cast<const void *>(sweep_persistent<false>), reinterpret_cast<const void *>(sweep_persistent<true>)},
         {reinterpret_cast<const void *>(sweep_xcd<false>), reinterpret_cast<const void *>(sweep_xcd<true>)},
@@ -1798,6 +1805,13 @@ uint32_t coop_blocks(const dy_xpbd_s *x, int override_blocks, int threads, int m
 int assign_by_rounds(dy_xpbd_s *x, hipStream_t st, const Cons &cv, const float *im) {
     uint32_t h[kMWords];
     for (int pass = 0; pass < 2; ++pass) {
+        const uint32_t cap = x->cap + x->jcap;
+        list_rank<<<grid_for(2u * cap), kSolveThreads, 0, st>>>(x->adj, x->own, x->off.p, x->deg.p, x->meta, x->cstat,
+                                                                 x->slot, x->crank);
+        DY_LAUNCH_CHECK();
+        list_link<<<grid_for(cap), kSolveThreads, 0, st>>>(cv, x->meta, im, x->off.p, x->deg.p, x->slot, x->crank,
+                                                            x->lrec, x->pending, x->fr0, x->meta + kMFcnt);
+        DY_LAUNCH_CHECK();
         DY_TRY(hipMemcpyAsync(h, x->meta, sizeof(h), hipMemcpyDeviceToHost, st));
         DY_TRY(hipStreamSynchronize(st));
         const uint32_t nc = h[kMNc];
@@ -1828,12 +1842,6 @@ int assign_by_rounds(dy_xpbd_s *x, hipStream_t st, const Cons &cv, const float *
             // The reference's serial path: re-rank in contact order and rerun.
             round_control<<<1, 1, 0, st>>>(x->meta, 0, exceeded ? 2 : 1);
             DY_LAUNCH_CHECK();
-            list_rank<<<grid_for(2u * nc), kSolveThreads, 0, st>>>(x->adj, x->own, x->off.p, x->deg.p, x->meta,
-                                                                   x->slot, x->crank);
-            DY_LAUNCH_CHECK();
-            list_link<<<grid_for(nc), kSolveThreads, 0, st>>>(cv, x->meta, im, x->off.p, x->deg.p, x->slot, x->crank,
-                                                              x->lrec, x->pending, x->fr0, x->meta + kMFcnt, x->fq);
-            DY_LAUNCH_CHECK();
             continue;
         }
         if (h[kMAssigned] != nc) return DY_ERR_INTERNAL;
@@ -1863,8 +1871,8 @@ int dy_xpbd_create(dy_stream_t s, int n_iters, uint32_t max_contacts, float fric
     x->mu = friction;
     x->cap = max_contacts;
     hipError_t e = alloc_constraint_bufs(x, max_contacts);
-    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&x->meta_block), kMetaBlock);
-    if (e == hipSuccess) e = place_meta(x, hs(s));
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&x->meta), kMWords * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMemsetAsync(x->meta, 0, kMWords * sizeof(uint32_t), hs(s));
     if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&x->h_meta), kMWords * sizeof(uint32_t));
     if (e == hipSuccess) e = hipEventCreateWithFlags(&x->ev_meta, hipEventDisableTiming);
     if (e == hipSuccess) e = hipStreamSynchronize(hs(s));
@@ -1918,7 +1926,7 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
     DY_TRY_STATUS(x->deg.ensure(nb));
     DY_TRY_STATUS(x->off.ensure(nb));
     DY_TRY_STATUS(x->fill.ensure(nb));
-    DY_TRY_STATUS(x->used.ensure(nb));
+    DY_TRY_STATUS(x->used.ensure(2 * static_cast<size_t>(nb)));
     DY_TRY_STATUS(x->ver.ensure(nb));
     DY_TRY_STATUS(x->dyn.ensure(4 * static_cast<size_t>(nb)));
     DY_TRY_STATUS(x->sta.ensure(2 * static_cast<size_t>(nb)));
@@ -1927,8 +1935,8 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
     uint32_t top = nb > ncap ? nb : ncap;
     if (top < kMWords + kMaxColours + 1u) top = kMWords + kMaxColours + 1u;
     solve_prep<<<grid_for(top), kSolveThreads, 0, st>>>(*bv, cv->n, cap, nj, x->force_serial, x->deg.p, x->fill.p,
-                                                         x->used.p, x->ver.p, x->lam, x->hist, x->meta, x->dyn.p,
-                                                         x->sta.p);
+                                                         x->used.p, x->ver.p, x->lam, x->flow, x->hist, x->meta,
+                                                         x->dyn.p, x->sta.p);
     DY_LAUNCH_CHECK();
     if (nj) {
         joint_pack<<<ceil_div(nj, 256), 256, 0, st>>>(*jv, nb, x->jpk, x->jend, x->meta);
@@ -1941,33 +1949,30 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
     DY_LAUNCH_CHECK();
     DY_TRY_STATUS(scan_exclusive(st, x->deg.p, x->off.p, nb, x->meta + kMDyn, x->scan_tmp.p));
     solve_fill<<<grid_for(ncap), kSolveThreads, 0, st>>>(cs, x->meta, bv->inv_mass, x->off.p, x->fill.p, x->adj,
-                                                          x->own);
+                                                          x->own, x->cstat, x->state);
     DY_LAUNCH_CHECK();
-    list_rank<<<grid_for(2u * ncap), kSolveThreads, 0, st>>>(x->adj, x->own, x->off.p, x->deg.p, x->meta, x->slot,
-                                                              x->crank);
-    DY_LAUNCH_CHECK();
-    list_link<<<grid_for(ncap), kSolveThreads, 0, st>>>(cs, x->meta, bv->inv_mass, x->off.p, x->deg.p, x->slot,
-                                                         x->crank, x->lrec, x->pending, x->fr0, x->meta + kMFcnt,
-                                                         x->fq);
-    DY_LAUNCH_CHECK();
-
     const int J = nj ? 1 : 0;
     bool coop = x->path == 0 && !x->coop_refused && x->coop_assign_max > 0 && x->coop_sweep_max[J] > 0;
     if (x->timing) DY_TRY(hipEventRecord(x->ev[0], st));
     if (coop) {
-        AssignBufs B{cs, bv->inv_mass, x->adj, x->own, x->off.p, x->deg.p, x->slot, x->crank, x->lrec, x->fq,
-                     x->pending, x->used.p, x->state, x->fr0, x->fr1, x->meta, x->hist, x->boff, x->bfill, nb};
+        list_rank<<<grid_for(2u * ncap), kSolveThreads, 0, st>>>(x->adj, x->own, x->off.p, x->deg.p, x->meta, x->cstat,
+                                                                  x->slot, nullptr);
+        DY_LAUNCH_CHECK();
+        AssignBufs B{x->adj, x->own, x->off.p, x->deg.p, x->cstat, x->slot, x->flow, x->used.p, x->state, x->meta,
+                     x->hist, x->boff, x->bfill, nb};
         void *args[] = {&B};
-        // Participants on one XCD out of a launch with as many on every XCD:
-        // by default 16 workgroups of 256 threads per XCD on a 256-CU device,
-        // half the solver's usual share.  On the 32k-body frame 16 beat 8, 24
-        // and 32 (fewer workgroups meet at each round barrier).
-        const int assign_dflt = (x->device_cus / 16) * 256 / x->assign_threads;
-        uint32_t blocks = 8u * coop_blocks(x, x->assign_blocks_override > 0 ? x->assign_blocks_override : assign_dflt,
-                                           x->assign_threads, x->coop_assign_max);
-        if (blocks > static_cast<uint32_t>(x->coop_assign_max)) blocks = static_cast<uint32_t>(x->coop_assign_max);
-        if (try_coop_launch(reinterpret_cast<const void *>(assign_lists), dim3(blocks),
-                            dim3(static_cast<uint32_t>(x->assign_threads)), args, st) != hipSuccess) {
+        // A thread per body, as far as half of what the occupancy query promises
+        // holds them: the workgroups wait for each other, and the query has
+        // named one or two workgroups a CU more than were resident.
+        const bool one_xcd = nb <= kAssignOneXcd;
+        const uint32_t most = static_cast<uint32_t>(x->coop_assign_max > 1 ? x->coop_assign_max / 2 : 1);
+        uint32_t blocks = x->assign_blocks_override > 0 ? static_cast<uint32_t>(x->assign_blocks_override)
+                                                        : ceil_div(nb ? nb : 1u, static_cast<uint32_t>(x->assign_threads));
+        if (one_xcd) blocks *= 8u;  // an eighth of a launch runs on the XCD
+        if (blocks > most) blocks = most;
+        if (try_coop_launch(one_xcd ? reinterpret_cast<const void *>(assign_flow<true>)
+                                    : reinterpret_cast<const void *>(assign_flow<false>),
+                            dim3(blocks), dim3(static_cast<uint32_t>(x->assign_threads)), args, st) != hipSuccess) {
             x->coop_refused = true;
             coop = false;
         }

@@ -1,0 +1,80 @@
+"""Class assignment: every body's thread in lock step with its partners, on one
+XCD (few bodies) and over the chip, with one body a thread and several."""
+import numpy as np
+import pytest
+
+from dyphur_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _greedy(a, b, static, serial):
+    """Classes by definition: in priority order (JP) the lowest colour free on
+    both bodies, in index order one more than the bodies' levels."""
+    k = np.arange(len(a), dtype=np.uint64)
+    if serial:
+        order = np.arange(len(a))
+    else:
+        h = k.astype(np.uint32)
+        h ^= h >> np.uint32(16)
+        h *= np.uint32(0x85EBCA6B)
+        h ^= h >> np.uint32(13)
+        h *= np.uint32(0xC2B2AE35)
+        h ^= h >> np.uint32(16)
+        order = np.argsort((h.astype(np.uint64) << np.uint64(32)) | k)[::-1]
+    used = [0] * len(static)
+    out = np.zeros(len(a), np.uint32)
+    for c in order:
+        ends = [x for x in (a[c], b[c]) if not static[x]]
+        if serial:
+            out[c] = max([used[x] for x in ends], default=0)
+            for x in ends:
+                used[x] = int(out[c]) + 1
+        else:
+            m = 0
+            for x in ends:
+                m |= used[x]
+            out[c] = (~m & (m + 1)).bit_length() - 1
+            for x in ends:
+                used[x] |= 1 << int(out[c])
+    return out
+
+
+@pytest.mark.parametrize("n,nc,blocks,serial", [
+    (64, 250, 0, False), (64, 257, 0, False), (1000, 3000, 0, False), (1000, 3000, 1, False), (1000, 900, 0, True),
+    (16384, 40001, 0, False), (16385, 40001, 0, False), (16385, 20000, 3, False), (16385, 9000, 2, True),
+])
+def test_classes_match_greedy(gpu, monkeypatch, n, nc, blocks, serial):
+    """Random contacts over n bodies (a tenth static; contacts between two
+    static bodies among them): both sides of the one-XCD line, of the
+    256-contact line, and with several bodies a thread."""
+    if blocks:
+        monkeypatch.setenv("DYPHUR_ASSIGN_BLOCKS", str(blocks))
+    print(f"[assign] n={n} nc={nc} blocks={blocks} serial={serial}", flush=True)
+    rng = np.random.default_rng(n + nc)
+    a = rng.integers(0, n, nc).astype(np.uint32)
+    b = ((a + rng.integers(1, n, nc)) % n).astype(np.uint32)
+    a.sort()  # grouped by the first body, as the broadphase lists them
+    b = np.where(a == b, (b + 1) % n, b).astype(np.uint32)
+    static = rng.random(n) < 0.1
+    sc = scenes.random_mixed(n - 1, seed=1, extent=(40, 40, 40))
+    sc.mass = np.where(static, 0.0, np.maximum(sc.mass, 1.0)).astype(np.float32)
+    sc.flags = np.where(static, scenes.FLAG_STATIC, 0).astype(np.uint32)
+    s = gpu.Stream()
+    db = gpu.DeviceBodies(sc, s)
+    solver = gpu.XpbdSolver(s, 2, nc, 0.5)
+    solver.set_force_serial(serial)
+    z = np.zeros(nc, np.float32)
+    arrays = [gpu.DeviceArray.from_numpy(v, s) for v in (a, b, z, z, z, z, z, z, z)]
+    count = gpu.DeviceArray.from_numpy(np.array([nc], np.uint32), s)
+    cv = gpu.ContactView()
+    for name, arr in zip(("body_a", "body_b", "pos_x", "pos_y", "pos_z", "norm_x", "norm_y", "norm_z", "depth"), arrays):
+        setattr(cv, name, arr.ptr)
+    cv.n, cv.capacity = count.ptr, nc
+    solver.solve(s, cv, db, sc.dt)
+    st = solver.stats()
+    used_serial = serial or nc <= 256
+    ref = _greedy(a, b, static, used_serial)
+    assert bool(st["used_serial"]) == used_serial
+    assert st["n_constraints"] == nc and st["n_classes"] == ref.max() + 1
+    assert np.array_equal(solver.classes(s, nc), ref)
