@@ -518,7 +518,9 @@ DY_HD bool project_contact(const ContactIn &c, BodyState &A, BodyState &B, float
 // project_contact forms left to right (w, the relative velocities, wt) are
 // formed on both lanes in the same order from exchanged terms, so every value
 // is bit-equal to project_contact's.  Every branch around an exchange depends
-// on shared values only, so the two lanes always take it together.
+// on shared values only, so the two lanes always take it together.  What body B
+// gets with the opposite sign takes it on the factor dl, jn or jt (products are
+// rounded the same with either sign), so both sides run the same instructions.
 template <class Xchg>
 DY_HD void project_contact_pair(const ContactIn &c, BodyState &S, uint32_t side, float mu, float &lam, float dt,
                                 Xchg &&pair_xchg) {
@@ -538,13 +540,9 @@ DY_HD void project_contact_pair(const ContactIn &c, BodyState &S, uint32_t side,
     if (w < 1e-10f) return;
     const float dl = rem / w;
     lam += rem;
-    if (side == 0u) {
-        if (wa != 0.f) { S.px += wa * dl * nx; S.py += wa * dl * ny; S.pz += wa * dl * nz; }
-        rotate_by(S, dl * kx, dl * ky, dl * kz);
-    } else {
-        if (wb != 0.f) { S.px -= wb * dl * nx; S.py -= wb * dl * ny; S.pz -= wb * dl * nz; }
-        rotate_by(S, -dl * kx, -dl * ky, -dl * kz);
-    }
+    const float dls = side ? -dl : dl;
+    if (ws != 0.f) { S.px += ws * dls * nx; S.py += ws * dls * ny; S.pz += ws * dls * nz; }
+    rotate_by(S, dls * kx, dls * ky, dls * kz);
     {
         const float vsx = S.vx + S.wy * rz - S.wz * ry;
         const float vsy = S.vy + S.wz * rx - S.wx * rz;
@@ -559,13 +557,9 @@ DY_HD void project_contact_pair(const ContactIn &c, BodyState &S, uint32_t side,
             float gx, gy, gz;
             inv_inertia_world(S, cx, cy, cz, gx, gy, gz);
             if (ws != 0.f) {
-                if (side == 0u) {
-                    S.vx += wa * jn * nx; S.vy += wa * jn * ny; S.vz += wa * jn * nz;
-                    S.wx += jn * gx; S.wy += jn * gy; S.wz += jn * gz;
-                } else {
-                    S.vx -= wb * jn * nx; S.vy -= wb * jn * ny; S.vz -= wb * jn * nz;
-                    S.wx -= jn * gx; S.wy -= jn * gy; S.wz -= jn * gz;
-                }
+                const float js = side ? -jn : jn;
+                S.vx += ws * js * nx; S.vy += ws * js * ny; S.vz += ws * js * nz;
+                S.wx += js * gx; S.wy += js * gy; S.wz += js * gz;
             }
         }
     }
@@ -596,13 +590,9 @@ DY_HD void project_contact_pair(const ContactIn &c, BodyState &S, uint32_t side,
                 float jt = tl / wt;
                 jt = fminf(jt, mu * jcap);
                 if (ws != 0.f) {
-                    if (side == 0u) {
-                        S.vx -= wa * jt * tx; S.vy -= wa * jt * ty; S.vz -= wa * jt * tz;
-                        S.wx -= jt * fx; S.wy -= jt * fy; S.wz -= jt * fz;
-                    } else {
-                        S.vx += wb * jt * tx; S.vy += wb * jt * ty; S.vz += wb * jt * tz;
-                        S.wx += jt * fx; S.wy += jt * fy; S.wz += jt * fz;
-                    }
+                    const float js = side ? jt : -jt;
+                    S.vx += ws * js * tx; S.vy += ws * js * ty; S.vz += ws * js * tz;
+                    S.wx += js * fx; S.wy += js * fy; S.wz += js * fz;
                 }
             }
         }

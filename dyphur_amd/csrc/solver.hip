@@ -56,6 +56,9 @@ constexpr uint32_t kMaxGridBlocks = 1024;  // grid-stride kernels over capacity-
 // Bodies up to which assign_flow runs on one XCD (one XCD against the chip, mid-run piles: 2 000 bodies 38 against
 // 58 us, 5 000 54 / 81, 8 000 65 / 90, 12 000 80 / 101, 20 000 89 / 89, 32 768 250 / 98).
 constexpr uint32_t kAssignOneXcd = 16384;
+// The same line for sweep_first (one XCD against the chip: 1 024 boxes 45 against 52 us, 5 000 bodies 90 / 108,
+// 32 768 189 / 169, 98 305 457 / 254).
+constexpr uint32_t kSweepOneXcd = 16384;
 constexpr uint32_t kSweepXcc = 0;         // the XCD whose workgroups run the assignment and the sweep
 
 // Solver metadata (device words).  solve_prep zeroes all but kMErr, which
@@ -83,7 +86,8 @@ enum : uint32_t {
     kMRegMotor = 28,     // 2 words: check-in of joint_motors_xcd
     kMBarMotor = 30,     // 2 words: barrier of joint_motors_xcd
     kMRegAssign = 32,    // 2 words: check-in of assign_flow on one XCD
-    kMWords = 34,
+    kMRegFirst = 34,     // 2 words: check-in of sweep_first on one XCD
+    kMWords = 36,
 };
 constexpr uint32_t kErrBarrier = 2u, kErrCapacity = 4u, kErrAssign = 8u, kErrFlow = 16u, kErrJoint = 32u;
 
@@ -116,14 +120,30 @@ __device__ __forceinline__ void gather_body(const dy_body_view &bv, uint32_t i, 
     sta[2 * i + 1] = make_float4(bv.iI_xy[i], bv.iI_xz[i], bv.iI_yz[i], 0.f);
 }
 
+// A body's state as sweep_first hands it from contact to contact: 13 words of
+// (float, tag << 32), tag = contacts of the first iteration applied to it, in
+// the order of BodyState; one 128-byte line a body.
+constexpr uint32_t kBodyWords = 16, kBodyFloats = 13;
+__device__ __forceinline__ void gather_words(const dy_body_view &bv, uint32_t i, uint64_t *__restrict__ bw,
+                                             float4 *__restrict__ sta) {
+    const float v[kBodyFloats] = {bv.pos_x[i], bv.pos_y[i], bv.pos_z[i], bv.rot_w[i], bv.rot_x[i],
+                                  bv.rot_y[i], bv.rot_z[i], bv.vel_x[i], bv.vel_y[i], bv.vel_z[i],
+                                  bv.ang_x[i], bv.ang_y[i], bv.ang_z[i]};
+    ulonglong2 *w = reinterpret_cast<ulonglong2 *>(bw + static_cast<size_t>(i) * kBodyWords);
+#pragma unroll
+    for (uint32_t k = 0; k < kBodyFloats; k += 2u)
+        w[k / 2u] = make_ulonglong2(__float_as_uint(v[k]), k + 1u < kBodyFloats ? __float_as_uint(v[k + 1u]) : 0u);
+    sta[2 * i + 0] = make_float4(bv.inv_mass[i], bv.iI_xx[i], bv.iI_yy[i], bv.iI_zz[i]);
+    sta[2 * i + 1] = make_float4(bv.iI_xy[i], bv.iI_xz[i], bv.iI_yz[i], 0.f);
+}
+
 // Per-solve reset (per-body counters and masks, per-constraint lambdas, the
-// metadata) and the bodies' AoS records.
+// metadata) and the bodies' AoS records (their words when bw is given).
 __global__ void solve_prep(dy_body_view bv, const uint32_t *__restrict__ ncp, uint32_t cap, uint32_t nj,
                            int force_serial, uint32_t *__restrict__ deg, uint32_t *__restrict__ fill,
                            uint64_t *__restrict__ used, uint32_t *__restrict__ ver, float *__restrict__ lam,
                            FlowWord *__restrict__ flow, uint32_t *__restrict__ hist, uint32_t *__restrict__ meta,
-                           float4 *__restrict__ dyn,
-                           float4 *__restrict__ sta) {
+                           float4 *__restrict__ dyn, float4 *__restrict__ sta, uint64_t *__restrict__ bw) {
     const uint32_t nb = bv.n;
     const uint32_t n_raw = *ncp;
     const uint32_t nc = n_raw < cap ? n_raw : cap;
@@ -139,7 +159,8 @@ __global__ void solve_prep(dy_body_view bv, const uint32_t *__restrict__ ncp, ui
             used[i] = 0;
             used[nb + i] = 0;
             ver[i] = 0;
-            gather_body(bv, i, dyn, sta);
+            if (bw) gather_words(bv, i, bw, sta);
+            else gather_body(bv, i, dyn, sta);
         }
         if (i < ncon) {
             lam[i] = 0.f;
@@ -1377,16 +1398,169 @@ __global__ __launch_bounds__(1024) void sweep_flow(uint32_t n_iters, CRec rec, c
     }
 }
 
+// A body's words, read between kernels.
+__device__ __forceinline__ BodyState words_state(const uint64_t *__restrict__ bw, uint32_t i, uint32_t &tag) {
+    const ulonglong2 *w = reinterpret_cast<const ulonglong2 *>(bw + static_cast<size_t>(i) * kBodyWords);
+    float v[kBodyFloats + 1];
+#pragma unroll
+    for (uint32_t k = 0; k < kBodyFloats; k += 2u) {
+        const ulonglong2 e = w[k / 2u];
+        v[k] = __uint_as_float(static_cast<uint32_t>(e.x));
+        v[k + 1u] = __uint_as_float(static_cast<uint32_t>(e.y));
+        if (k == 0) tag = static_cast<uint32_t>(e.x >> 32);
+    }
+    BodyState s{};
+    s.px = v[0]; s.py = v[1]; s.pz = v[2]; s.qw = v[3]; s.qx = v[4]; s.qy = v[5]; s.qz = v[6];
+    s.vx = v[7]; s.vy = v[8]; s.vz = v[9]; s.wx = v[10]; s.wy = v[11]; s.wz = v[12];
+    return s;
+}
+
+// The words while they move: 16-byte accesses past the L1, each 64-bit half a
+// single-copy one that carries its own tag.
+__device__ __forceinline__ u32x4 ld_words2(const uint64_t *p) {
+    u32x4 v;
+    asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(v) : "v"(p) : "memory");
+    return v;
+}
+__device__ __forceinline__ void ld_words_rest(const uint64_t *p, u32x4 (&v)[7]) {
+    asm volatile("global_load_dwordx4 %0, %6, off offset:16 sc1\n\tglobal_load_dwordx4 %1, %6, off offset:32 sc1\n\t"
+                 "global_load_dwordx4 %2, %6, off offset:48 sc1\n\tglobal_load_dwordx4 %3, %6, off offset:64 sc1\n\t"
+                 "global_load_dwordx4 %4, %6, off offset:80 sc1\n\tglobal_load_dwordx4 %5, %6, off offset:96 sc1\n\t"
+                 "s_waitcnt vmcnt(0)"
+                 : "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]) : "v"(p) : "memory");
+}
+// The other lane's v of a pair of lanes: a permutation within four lanes.
+__device__ __forceinline__ float pair_other(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xb1, 0xf, 0xf, true));
+}
+// On one XCD a word only has to reach its L2.  A store of more than 8 bytes
+// reads its data one wait state after issue.
+template <bool ONE_XCD>
+__device__ __forceinline__ void st_words2(uint64_t *p, float a, float b, uint32_t tag) {
+    const u32x4 v = {__float_as_uint(a), tag, __float_as_uint(b), tag};
+    if (ONE_XCD) asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+    else asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+}
+
+// The first iteration of a contact-only dataflow sweep, a pair of lanes per
+// record as sweep_flow_pair.  The body's state goes from contact to contact
+// as words that carry their version: a lane reads its body until every word
+// has the version its contact waits for, so nothing is acknowledged before a
+// version is published and nothing is read again after it was seen.
+//
+// Bound by the chain of classes (15 on a settled stack of 1 024 boxes, 45 on a
+// pile of 32 768 bodies): about 1.3 us of projection and 1.4 us of hand-over a
+// step.  Because the words need no cache of their own, the chip can take part;
+// the one-XCD form has the shorter hand-over until its lanes are short (see
+// kSweepOneXcd).  Against records handed over by acknowledged stores, a version
+// and a second read on one XCD: 1 024 boxes 65 -> 45 us, 5 000 bodies 122 -> 90,
+// 32 768 225 -> 169, 98 305 523 -> 254.  R records a wavefront: over the chip 16
+// (182 us) measured better than 32 (220) and 8 with twice the workgroups as 16.
+// Reading every word of a body that is one contact away (instead of two words
+// until they match) was slower from 32 768 bodies on (216 us).
+template <bool ONE_XCD>
+__global__ __launch_bounds__(512) void sweep_first(CRec rec, const uint4 *__restrict__ rseq, float *__restrict__ lam,
+                                                   uint64_t *bw, const float4 *__restrict__ sta, float mu, float dt,
+                                                   uint32_t *meta) {
+    uint32_t *err = meta + kMErr;
+    uint32_t bidx = blockIdx.x, nblk = gridDim.x;
+    if (ONE_XCD && !xcd_checkin(kSweepXcc, meta + kMRegFirst, err, kErrBarrier, bidx, nblk)) return;
+    if (meta[kMErr] & kErrAssign) return;
+    const uint32_t nc = meta[kMNc];
+    constexpr uint32_t R = ONE_XCD ? 32u : 16u;
+    const uint32_t nw = blockDim.x / 64u;
+    const uint32_t lane = lane_id(), side = lane & 1u;
+    for (uint32_t r0 = ((threadIdx.x >> 6) * nblk + bidx) * R; r0 < nc; r0 += nblk * nw * R) {
+        const uint32_t i = r0 + (lane >> 1);
+        bool todo = lane < 2u * R && i < nc;  // the same on both lanes of a pair
+        uint32_t x = 0, t = 0;
+        bool dyn_end = false;
+        float4 p0 = make_float4(0.f, 0.f, 0.f, 0.f), p1 = p0;
+        BodyState S{};
+        if (todo) {
+            const uint2 ab = rec.ab[i];
+            const uint4 sq = rseq[i];
+            p0 = rec.p0[i];
+            p1 = rec.p1[i];
+            x = side ? ab.y : ab.x;             // this lane's body
+            dyn_end = (side ? sq.w : sq.y) != 0u;  // a dynamic end: it waits and publishes
+            t = side ? sq.z : sq.x;
+            const float4 s0 = sta[2 * x], s1 = sta[2 * x + 1];
+            S.im = s0.x; S.ixx = s0.y; S.iyy = s0.z; S.izz = s0.w;
+            S.ixy = s1.x; S.ixz = s1.y; S.iyz = s1.z;
+        }
+        uint64_t *w = bw + static_cast<size_t>(x) * kBodyWords;
+        const bool live = contact_live(p1.z, 0.f);
+        bool have = false;
+        uint32_t spins = 0;
+        while (__ballot(todo)) {
+            if (todo && !have) {
+                u32x4 v[7];
+                v[0] = ld_words2(w);
+                if (!dyn_end || (v[0].y == t && v[0].w == t)) {
+                    ld_words_rest(w, v);
+                    bool all = v[6].y == t;
+#pragma unroll
+                    for (uint32_t k = 1; k < 6u; ++k) all = all && v[k].y == t && v[k].w == t;
+                    have = all || !dyn_end;
+                    auto f = [](uint32_t u) { return __uint_as_float(u); };
+                    S.px = f(v[0].x); S.py = f(v[0].z); S.pz = f(v[1].x); S.qw = f(v[1].z);
+                    S.qx = f(v[2].x); S.qy = f(v[2].z); S.qz = f(v[3].x); S.vx = f(v[3].z);
+                    S.vy = f(v[4].x); S.vz = f(v[4].z); S.wx = f(v[5].x); S.wy = f(v[5].z);
+                    S.wz = f(v[6].x);
+                }
+            }
+            // the exchange runs on every lane: a lane inside a short-circuit would read an inactive partner
+            const int partner = __builtin_amdgcn_mov_dpp(have ? 1 : 0, 0xb1, 0xf, 0xf, true);
+            const bool ready = todo && have && partner != 0;
+            if (ready) {
+                if (live) {
+                    float l = 0.f;
+                    const ContactIn ci{p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z};
+                    project_contact_pair(ci, S, side, mu, l, dt, [](float v) { return pair_other(v); });
+                    if (side == 0u) {
+                        lam[i] = l;
+                        if (contact_live(p1.z, l)) atomicOr(&meta[kMLive], 1u);
+                    }
+                }
+                if (dyn_end) {
+                    st_words2<ONE_XCD>(w, S.px, S.py, t + 1u);
+                    st_words2<ONE_XCD>(w + 2, S.pz, S.qw, t + 1u);
+                    st_words2<ONE_XCD>(w + 4, S.qx, S.qy, t + 1u);
+                    st_words2<ONE_XCD>(w + 6, S.qz, S.vx, t + 1u);
+                    st_words2<ONE_XCD>(w + 8, S.vy, S.vz, t + 1u);
+                    st_words2<ONE_XCD>(w + 10, S.wx, S.wy, t + 1u);
+                    st_words2<ONE_XCD>(w + 12, S.wz, 0.f, t + 1u);
+                }
+                todo = false;
+            }
+            if (__ballot(ready)) {
+                spins = 0;
+                continue;
+            }
+            __builtin_amdgcn_s_sleep(1);
+            if (++spins > kGridSpinLimit) {
+                if (lane == 0) atomicOr(err, kErrFlow);
+                return;
+            }
+            if ((spins & 255u) == 0u && (ld_agent(err) & kErrFlow)) return;
+        }
+    }
+}
+
 // Contact-only dataflow sweep with a pair of lanes per record (lanes 2k and
 // 2k + 1 of a wave take record i0 + k, one body each, project_contact_pair):
 // each lane polls, loads, renormalises, stores and publishes its own body,
 // so a pass of the projection is about half as long.  Otherwise sweep_flow.
+// With `bw`, sweep_first has done iteration 0: nothing is left to do unless a
+// contact is still live, and then the bodies' records are made from their words.
 __global__ __launch_bounds__(1024) void sweep_flow_pair(uint32_t n_iters, CRec rec, const uint4 *__restrict__ rseq,
                                                         float *__restrict__ lam, float4 *__restrict__ dyn,
                                                         const float4 *__restrict__ sta, uint32_t *ver, float mu,
                                                         float dt, uint32_t *meta,
-                                                        const float4 *__restrict__ /* joints: none */) {
+                                                        const uint64_t *__restrict__ bw, uint32_t nb) {
     uint32_t *err = meta + kMErr;
+    if (bw && meta[kMLive] == 0u) return;
     uint32_t bidx = 0, nblk = 0;
     if (!xcd_checkin(kSweepXcc, meta + kMRegSweep, err, kErrBarrier, bidx, nblk)) return;
     if (meta[kMErr] & kErrAssign) return;
@@ -1395,8 +1569,16 @@ __global__ __launch_bounds__(1024) void sweep_flow_pair(uint32_t n_iters, CRec r
     const uint32_t lane = lane_id(), side = lane & 1u;
     const uint32_t wave_rec0 = (bidx * blockDim.x + (threadIdx.x & ~63u)) / 2u;
     uint32_t gen = 0;
-    for (uint32_t it = 0; it < n_iters; ++it) {
-        if (it == 1) {
+    if (bw) {
+        for (uint32_t i = bidx * blockDim.x + threadIdx.x; i < nb; i += nblk * blockDim.x) {
+            uint32_t tag;
+            store_aos(dyn, i, words_state(bw, i, tag), 0u);
+            ver[i] = tag;
+        }
+        if (!xcd_barrier(meta + kMBarSweep, gen, nblk, err, kErrBarrier)) return;
+    }
+    for (uint32_t it = bw ? 1u : 0u; it < n_iters; ++it) {
+        if (it == 1 && !bw) {
             if (!xcd_barrier(meta + kMBarSweep, gen, nblk, err, kErrBarrier)) return;
             if (ld_agent(&meta[kMLive]) == 0u) return;
         }
@@ -1534,10 +1716,22 @@ __global__ __launch_bounds__(1024) void sweep_flow_lanes(uint32_t n_iters, CRec 
     }
 }
 
-// Back to the SoA view, bringing every body to n_iters renormalisations.
-__global__ void scatter_bodies(dy_body_view bv, const float4 *__restrict__ dyn, uint32_t n_iters) {
+// Back to the SoA view, bringing every body to n_iters renormalisations.  With
+// `bw`, from the bodies' words unless later iterations moved on to the records.
+__global__ void scatter_bodies(dy_body_view bv, const float4 *__restrict__ dyn, uint32_t n_iters,
+                               const uint64_t *__restrict__ bw, const uint32_t *__restrict__ meta) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= bv.n) return;
+    if (bw && (meta[kMLive] == 0u || n_iters < 2u)) {
+        uint32_t tag;
+        BodyState S = words_state(bw, i, tag);
+        for (uint32_t r = 0; r < n_iters; ++r) renormalise(S.qw, S.qx, S.qy, S.qz);
+        bv.pos_x[i] = S.px; bv.pos_y[i] = S.py; bv.pos_z[i] = S.pz;
+        bv.rot_w[i] = S.qw; bv.rot_x[i] = S.qx; bv.rot_y[i] = S.qy; bv.rot_z[i] = S.qz;
+        bv.vel_x[i] = S.vx; bv.vel_y[i] = S.vy; bv.vel_z[i] = S.vz;
+        bv.ang_x[i] = S.wx; bv.ang_y[i] = S.wy; bv.ang_z[i] = S.wz;
+        return;
+    }
     const float4 d0 = dyn[4 * i], d1 = dyn[4 * i + 1], d2 = dyn[4 * i + 2], d3 = dyn[4 * i + 3];
     float qw = d0.w, qx = d1.x, qy = d1.y, qz = d1.z;
     for (uint32_t r = __float_as_uint(d3.y); r < n_iters; ++r) renormalise(qw, qx, qy, qz);
@@ -1545,6 +1739,13 @@ __global__ void scatter_bodies(dy_body_view bv, const float4 *__restrict__ dyn, 
     bv.rot_w[i] = qw; bv.rot_x[i] = qx; bv.rot_y[i] = qy; bv.rot_z[i] = qz;
     bv.vel_x[i] = d1.w; bv.vel_y[i] = d2.x; bv.vel_z[i] = d2.y;
     bv.ang_x[i] = d2.z; bv.ang_y[i] = d2.w; bv.ang_z[i] = d3.x;
+}
+
+// The bodies' records from their words (a sweep that does not take words runs after all).
+__global__ void words_to_records(const uint64_t *__restrict__ bw, uint32_t nb, float4 *__restrict__ dyn) {
+    const uint32_t i = grid_tid();
+    uint32_t tag;
+    if (i < nb) store_aos(dyn, i, words_state(bw, i, tag), 0u);
 }
 
 // Class of each contact id (for dy_xpbd_download_classes).
@@ -1576,6 +1777,7 @@ struct dy_xpbd_s {
     DevBuf<uint32_t> deg, off, fill, scan_tmp, ver;
     DevBuf<uint64_t> used;
     DevBuf<float4> dyn, sta;
+    DevBuf<uint64_t> bw;
     // Metadata of the last solve, copied back asynchronously into pinned
     // memory; ev_meta completes when the copy has landed.
     uint32_t *h_meta = nullptr;
@@ -1586,7 +1788,7 @@ struct dy_xpbd_s {
     // Co-resident workgroup limits of the cooperative kernels, [0] contacts
     // only, [1] the variants that also solve joints.
     int coop_assign_max = 0, coop_sweep_max[2] = {0, 0}, coop_xcd_max[2] = {0, 0}, coop_flow_max[2] = {0, 0},
-        coop_lanes_max[2] = {0, 0}, coop_pair_max = 0, coop_motor_max = 0, device_cus = 0;
+        coop_lanes_max[2] = {0, 0}, coop_pair_max = 0, coop_first_max = 0, coop_motor_max = 0, device_cus = 0;
     int sweep_pair = 1;     // contact-only dataflow sweeps use sweep_flow_pair (DYPHUR_SWEEP_PAIR=0: sweep_flow)
     int pair_threads = 512;  // its workgroup size (DYPHUR_SWEEP_PAIR_THREADS)
     // Constraint capacity (contacts + joints) of the constraint-indexed
@@ -1727,7 +1929,7 @@ void xp_free(dy_xpbd_s *x) {
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     x->deg.release(); x->off.release(); x->fill.release(); x->scan_tmp.release(); x->ver.release();
-    x->used.release(); x->dyn.release(); x->sta.release();
+    x->used.release(); x->dyn.release(); x->sta.release(); x->bw.release();
 }
 
 int env_int(const char *name, int dflt) {
@@ -1788,6 +1990,11 @@ int query_coop(dy_xpbd_s *x) {
     DY_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(sweep_flow_pair),
                                                         x->pair_threads, 0));
     x->coop_pair_max = per_cu * x->device_cus;
+    DY_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(sweep_first<false>),
+                                                        x->pair_threads, 0));
+    DY_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_xcd, reinterpret_cast<const void *>(sweep_first<true>),
+                                                        x->pair_threads, 0));
+    x->coop_first_max = (per_cu < per_cu_xcd ? per_cu : per_cu_xcd) * x->device_cus;
     return DY_OK;
 }
 
@@ -1932,11 +2139,17 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
     DY_TRY_STATUS(x->sta.ensure(2 * static_cast<size_t>(nb)));
     DY_TRY_STATUS(x->scan_tmp.ensure(scan_tmp_words(nb > ncap + 66u ? nb : ncap + 66u)));
     x->last_nb = nb;
+    const int J = nj ? 1 : 0;
+    bool coop = x->path == 0 && !x->coop_refused && x->coop_assign_max > 0 && x->coop_sweep_max[J] > 0;
+    // contact-only dataflow sweeps: a pair of lanes per record, the first iteration by sweep_first
+    const bool pair = x->sweep_mode == 2 && !J && x->sweep_pair && x->coop_pair_max > 0 && x->coop_first_max > 0;
+    bool words = coop && pair;
+    if (words) DY_TRY_STATUS(x->bw.ensure(static_cast<size_t>(kBodyWords) * nb));
     uint32_t top = nb > ncap ? nb : ncap;
     if (top < kMWords + kMaxColours + 1u) top = kMWords + kMaxColours + 1u;
     solve_prep<<<grid_for(top), kSolveThreads, 0, st>>>(*bv, cv->n, cap, nj, x->force_serial, x->deg.p, x->fill.p,
                                                          x->used.p, x->ver.p, x->lam, x->flow, x->hist, x->meta,
-                                                         x->dyn.p, x->sta.p);
+                                                         x->dyn.p, x->sta.p, words ? x->bw.p : nullptr);
     DY_LAUNCH_CHECK();
     if (nj) {
         joint_pack<<<ceil_div(nj, 256), 256, 0, st>>>(*jv, nb, x->jpk, x->jend, x->meta);
@@ -1951,8 +2164,6 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
     solve_fill<<<grid_for(ncap), kSolveThreads, 0, st>>>(cs, x->meta, bv->inv_mass, x->off.p, x->fill.p, x->adj,
                                                           x->own, x->cstat, x->state);
     DY_LAUNCH_CHECK();
-    const int J = nj ? 1 : 0;
-    bool coop = x->path == 0 && !x->coop_refused && x->coop_assign_max > 0 && x->coop_sweep_max[J] > 0;
     if (x->timing) DY_TRY(hipEventRecord(x->ev[0], st));
     if (coop) {
         list_rank<<<grid_for(2u * ncap), kSolveThreads, 0, st>>>(x->adj, x->own, x->off.p, x->deg.p, x->meta, x->cstat,
@@ -2022,11 +2233,39 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
     const float4 *jpkv = x->jpk;
     if (x->timing) DY_TRY(hipEventRecord(x->ev[2], st));
     bool swept = iters == 0;
+    const bool gathered = words;  // solve_prep wrote words
+    if (words && (swept || !coop || !flow)) words = false;
+    if (words) {
+        // a workgroup per CU, of the chip or of the one XCD (an eighth of the launch)
+        const bool one_xcd = nb <= kSweepOneXcd;
+        const int dflt = one_xcd ? x->device_cus / 8 : x->device_cus;
+        uint32_t blocks = coop_blocks(x, x->sweep_blocks_override > 0 ? x->sweep_blocks_override : dflt, x->pair_threads,
+                                      x->coop_first_max);
+        if (one_xcd) blocks *= 8u;
+        if (blocks > static_cast<uint32_t>(x->coop_first_max)) blocks = static_cast<uint32_t>(x->coop_first_max);
+        const uint4 *rseqv = x->rseq;
+        float *lamv = x->lam;
+        uint64_t *bwv = x->bw.p;
+        const float4 *stav = x->sta.p;
+        float muv = x->mu, dtv = dt;
+        uint32_t *metav = x->meta;
+        void *args[] = {&rec, &rseqv, &lamv, &bwv, &stav, &muv, &dtv, &metav};
+        if (try_coop_launch(one_xcd ? reinterpret_cast<const void *>(sweep_first<true>)
+                                    : reinterpret_cast<const void *>(sweep_first<false>),
+                            dim3(blocks), dim3(static_cast<uint32_t>(x->pair_threads)), args, st) != hipSuccess) {
+            x->coop_refused = true;
+            coop = false;
+            words = false;
+        }
+    }
+    if (gathered && !words) {
+        words_to_records<<<ceil_div(nb ? nb : 1u, 256), 256, 0, st>>>(x->bw.p, nb, x->dyn.p);
+        DY_LAUNCH_CHECK();
+    }
+    if (words && iters == 1u) swept = true;
     if (!swept && coop && flow) {
-        // contact-only: a pair of lanes per record, one workgroup of
-        // pair_threads per CU of the XCD by default (the measured best on the
-        // 32k-body frame: 32 x 512 against 16..48 x 256..1024)
-        const bool pair = x->sweep_mode == 2 && !J && x->sweep_pair && x->coop_pair_max > 0;
+        // one workgroup of pair_threads per CU of the XCD by default (the
+        // measured best on the 32k-body frame: 32 x 512 against 16..48 x 256..1024)
         const int threads = pair ? x->pair_threads : x->sweep_threads;
         const int cap = pair ? x->coop_pair_max : flow_max[J];
         uint32_t blocks = 8u * coop_blocks(x, x->sweep_blocks_override > 0 ? x->sweep_blocks_override
@@ -2041,7 +2280,11 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
         const float4 *stav = x->sta.p;
         uint32_t *verv = x->ver.p, *metav = x->meta;
         float muv = x->mu, dtv = dt;
-        void *args[] = {&iv, &rec, &rseqv, &lamv, &dynv, &stav, &verv, &muv, &dtv, &metav, &jpkv};
+        const uint64_t *bwv = words ? x->bw.p : nullptr;
+        uint32_t nbv = nb;
+        void *args_pair[] = {&iv, &rec, &rseqv, &lamv, &dynv, &stav, &verv, &muv, &dtv, &metav, &bwv, &nbv};
+        void *args_flow[] = {&iv, &rec, &rseqv, &lamv, &dynv, &stav, &verv, &muv, &dtv, &metav, &jpkv};
+        void **args = pair ? args_pair : args_flow;
         const void *fn;
         if (x->sweep_mode == 3)
             fn = J ? reinterpret_cast<const void *>(sweep_flow_lanes<true>)
@@ -2098,7 +2341,7 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
         DY_TRY(hipEventRecord(x->ev[3], st));
         x->ev_pending = true;
     }
-    scatter_bodies<<<ceil_div(nb, 256), 256, 0, st>>>(*bv, x->dyn.p, iters);
+    scatter_bodies<<<ceil_div(nb, 256), 256, 0, st>>>(*bv, x->dyn.p, iters, words ? x->bw.p : nullptr, x->meta);
     DY_LAUNCH_CHECK();
     DY_TRY(hipMemcpyAsync(x->h_meta, x->meta, kMWords * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
     DY_TRY(hipEventRecord(x->ev_meta, st));

@@ -40,6 +40,30 @@ def _greedy(a, b, static, serial):
     return out
 
 
+def _contacts(n, nc):
+    """Random contacts over n bodies, a tenth of them static, grouped by the
+    first body as the broadphase lists them."""
+    rng = np.random.default_rng(n + nc)
+    a = np.sort(rng.integers(0, n, nc)).astype(np.uint32)
+    b = ((a + rng.integers(1, n, nc)) % n).astype(np.uint32)
+    static = rng.random(n) < 0.1
+    sc = scenes.random_mixed(n - 1, seed=1, extent=(40, 40, 40))
+    sc.mass = np.where(static, 0.0, np.maximum(sc.mass, 1.0)).astype(np.float32)
+    sc.flags = np.where(static, scenes.FLAG_STATIC, 0).astype(np.uint32)
+    return a, b, static, sc
+
+
+def _view(gpu, s, a, b, fields):
+    names = ("body_a", "body_b", "pos_x", "pos_y", "pos_z", "norm_x", "norm_y", "norm_z", "depth")
+    arrays = [gpu.DeviceArray.from_numpy(np.ascontiguousarray(v), s) for v in (a, b, *fields)]
+    arrays.append(gpu.DeviceArray.from_numpy(np.array([len(a)], np.uint32), s))
+    cv = gpu.ContactView()
+    for name, arr in zip(names, arrays):
+        setattr(cv, name, arr.ptr)
+    cv.n, cv.capacity = arrays[-1].ptr, len(a)
+    return cv, arrays
+
+
 @pytest.mark.parametrize("n,nc,blocks,serial", [
     (64, 250, 0, False), (64, 257, 0, False), (1000, 3000, 0, False), (1000, 3000, 1, False), (1000, 900, 0, True),
     (16384, 40001, 0, False), (16385, 40001, 0, False), (16385, 20000, 3, False), (16385, 9000, 2, True),
@@ -51,26 +75,13 @@ def test_classes_match_greedy(gpu, monkeypatch, n, nc, blocks, serial):
     if blocks:
         monkeypatch.setenv("DYPHUR_ASSIGN_BLOCKS", str(blocks))
     print(f"[assign] n={n} nc={nc} blocks={blocks} serial={serial}", flush=True)
-    rng = np.random.default_rng(n + nc)
-    a = rng.integers(0, n, nc).astype(np.uint32)
-    b = ((a + rng.integers(1, n, nc)) % n).astype(np.uint32)
-    a.sort()  # grouped by the first body, as the broadphase lists them
-    b = np.where(a == b, (b + 1) % n, b).astype(np.uint32)
-    static = rng.random(n) < 0.1
-    sc = scenes.random_mixed(n - 1, seed=1, extent=(40, 40, 40))
-    sc.mass = np.where(static, 0.0, np.maximum(sc.mass, 1.0)).astype(np.float32)
-    sc.flags = np.where(static, scenes.FLAG_STATIC, 0).astype(np.uint32)
     s = gpu.Stream()
+    a, b, static, sc = _contacts(n, nc)
     db = gpu.DeviceBodies(sc, s)
     solver = gpu.XpbdSolver(s, 2, nc, 0.5)
     solver.set_force_serial(serial)
     z = np.zeros(nc, np.float32)
-    arrays = [gpu.DeviceArray.from_numpy(v, s) for v in (a, b, z, z, z, z, z, z, z)]
-    count = gpu.DeviceArray.from_numpy(np.array([nc], np.uint32), s)
-    cv = gpu.ContactView()
-    for name, arr in zip(("body_a", "body_b", "pos_x", "pos_y", "pos_z", "norm_x", "norm_y", "norm_z", "depth"), arrays):
-        setattr(cv, name, arr.ptr)
-    cv.n, cv.capacity = count.ptr, nc
+    cv, _keep = _view(gpu, s, a, b, [z] * 7)
     solver.solve(s, cv, db, sc.dt)
     st = solver.stats()
     used_serial = serial or nc <= 256
@@ -78,3 +89,40 @@ def test_classes_match_greedy(gpu, monkeypatch, n, nc, blocks, serial):
     assert bool(st["used_serial"]) == used_serial
     assert st["n_constraints"] == nc and st["n_classes"] == ref.max() + 1
     assert np.array_equal(solver.classes(s, nc), ref)
+
+
+@pytest.mark.parametrize("heavy", [False, True])
+@pytest.mark.parametrize("n,nc,iters,blocks", [
+    (40, 33, 10, 0), (300, 257, 1, 0), (300, 900, 10, 1), (16384, 40001, 3, 0), (16385, 40001, 3, 0), (16385, 40001, 2, 2),
+])
+def test_first_iteration_by_words_matches_records(gpu, monkeypatch, n, nc, iters, blocks, heavy):
+    """The sweep that hands bodies on as tagged words against the sweep over
+    acknowledged records, bit for bit.  Contacts between bodies of almost no
+    inverse mass stay live after the first iteration, so the later ones run."""
+    if blocks:
+        monkeypatch.setenv("DYPHUR_SWEEP_BLOCKS", str(blocks))
+    rng = np.random.default_rng(7)
+    a, b, static, sc = _contacts(n, nc)
+    if heavy:
+        big = (rng.random(n) < 0.3) & ~static
+        sc.mass[big] = 1e13
+        sc.inertia[np.ix_(big, [0, 4, 8])] = 1e13
+    normal = rng.normal(size=(3, nc))
+    normal /= np.linalg.norm(normal, axis=0)
+    depth = rng.uniform(-0.01, 0.05, nc)
+    at = sc.pos[a].T + rng.uniform(-0.3, 0.3, (3, nc))
+    fields = [v.astype(np.float32) for v in (*at, *normal, depth)]
+    got = []
+    for pair in ("1", "0"):
+        monkeypatch.setenv("DYPHUR_SWEEP_PAIR", pair)
+        print(f"[words] n={n} nc={nc} iters={iters} blocks={blocks} heavy={heavy} pair={pair}", flush=True)
+        s = gpu.Stream()
+        db = gpu.DeviceBodies(sc, s)
+        solver = gpu.XpbdSolver(s, iters, nc, 0.5)
+        cv, _keep = _view(gpu, s, a, b, fields)
+        for _ in range(2):
+            solver.solve(s, cv, db, sc.dt)
+        assert solver.stats()["n_constraints"] == nc
+        got.append(db.download(s))
+    for k in got[0]:
+        assert np.array_equal(np.asarray(got[0][k]).view(np.uint32), np.asarray(got[1][k]).view(np.uint32)), k
