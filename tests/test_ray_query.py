@@ -154,3 +154,44 @@ def test_gpu_ray_query_bitexact(gpu, oracle, case):
     t, body = gpu.ray_query(s, bp, sc.n, db, ds, np.stack(rays))
     assert np.array_equal(body, b_ref)
     assert np.array_equal(t.view(np.uint32), t_ref.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m,moved,axis", [(2, 40, False, False), (3, 4096, False, True), (300, 4095, True, False),
+                                            (300, 4096, True, True), (1500, 20000, True, False),
+                                            (20000, 1200, True, False), (2000, 5000, False, True)])
+def test_gpu_ray_query_teams_bitexact(gpu, oracle, n, m, moved, axis):
+    """Rays walked by teams, from the view's arrays and from records: bodies
+    that moved since the tree was built (hits before their box), rays along the
+    axes and from the boxes' own planes (slab distances that are no number),
+    long rays through many bodies and every t_max."""
+    rng = np.random.default_rng(n + m)
+    side = 1.2 * n ** (1 / 3)
+    sc = scenes.random_mixed(n - 1, seed=5, extent=(side, side, side))
+    print(f"[ray teams] n={n} rays={m} moved={moved} axis={axis}", flush=True)
+    o = rng.uniform(-side, side, (m, 3))
+    d = rng.uniform(-side, side, (m, 3)) + [0, side / 2, 0] - o
+    if axis:
+        keep = rng.integers(0, 3, m)
+        sign = np.where(rng.random(m) < 0.5, 1.0, -1.0)
+        d = np.zeros((m, 3))
+        d[np.arange(m), keep] = sign
+        o[: m // 2] = np.round(o[: m // 2] * 4) / 4
+    t_max = rng.choice([0.5, 3.0, 50.0, np.inf], m)
+    rays = np.hstack([o, d, t_max[:, None]]).astype(F32)
+    (_, _), w, b, osh = _oracle_query(oracle, sc, list(rays[:1]))
+    s = gpu.Stream()
+    db = gpu.DeviceBodies(sc, s)
+    ds = gpu.DeviceShapes(sc, s)
+    bp = gpu.Broadphase(s, sc.n, sc.max_pairs)
+    bp.build_and_query(s, db, ds, sc.bounds)
+    if moved:
+        shift = rng.uniform(-0.3, 0.3, (3, sc.n)).astype(F32)
+        for k, f in enumerate(("pos_x", "pos_y", "pos_z")):
+            v = (db.download(s)[f] + shift[k]).astype(F32)
+            db.f[f].upload(v, s)
+            b.arr[f][:] = v
+    t_ref, b_ref = w.ray_query(b, osh, sc.n, rays)
+    t, body = gpu.ray_query(s, bp, sc.n, db, ds, rays)
+    assert np.array_equal(body, b_ref)
+    assert np.array_equal(t.view(np.uint32), t_ref.view(np.uint32))
