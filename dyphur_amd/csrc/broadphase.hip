@@ -1,9 +1,11 @@
 // broadphase.hip — LBVH broadphase for gfx950 (core/src/broadphase.cpp:101-365).
 //
 // Pipeline (all on one stream, no host synchronisation):
-//   1. morton_sort     one workgroup: 30-bit Morton codes of body centres, then a
-//                      stable 4-pass LSD radix sort of (code, body) — the same
-//                      order as the reference's sort of (code << 32 | body).
+//   1. rank_tiles, rank_merge, rank_scatter   30-bit Morton codes of body centres,
+//                      ordered by (code, body) through ranks — the same order as
+//                      the reference's sort of (code << 32 | body); past 262 144
+//                      bodies morton_sort_grid, a radix sort on one XCD (or
+//                      morton_sort, one workgroup).
 //   2. karras_build    one thread per internal node: children, parents, leaf
 //                      ranges and the depth-first "escape" links that make the
 //                      traversal stackless.
@@ -362,6 +364,111 @@ __global__ __launch_bounds__(kSgThreads) void morton_sort_grid(dy_body_view bv, 
         uint32_t *tk = sk; sk = dk; dk = tk;
         uint32_t *tv = sv; sv = dv; dv = tv;
     }
+}
+
+// Sort by ranks, the form for up to kRankMax bodies: ordinary launches over the
+// whole chip, no workgroup waits for another.
+//
+//  * rank_tiles: each 1 024-body tile, by counting for every key the tile's keys
+//    before it (64 rows x 256 columns a wavefront, four columns a broadcast LDS
+//    read), and the tile's keys in order.  One tile: that is the sort.
+//  * rank_merge: for every key of a tile, a binary search of another tile in
+//    LDS; one workgroup per (tile, group of tiles) sums its group's counts.
+//  * rank_scatter: a key's place is its place in its tile plus the groups' counts.
+//
+// Keys of equal code are ordered by body: a tile of earlier bodies counts its
+// equal keys, a tile of later ones does not.  The searches grow with the
+// square of the tiles.  Against the one-workgroup and one-XCD radix sorts (their
+// barriers and ballots on a few CUs): 64 bodies 18 -> 6 us, 1 025 23 -> 13,
+// 5 000 30 -> 14, 32 768 54 -> 19, 98 305 122 -> 41 (of it rank_merge 2.5, 3, 6
+// and 22); larger scenes keep the radix sort.  A key's count is of at most 8
+// tiles (kRankMax / kRankTile / kRankGroups), 16 bits.
+constexpr uint32_t kRankTile = 1024, kRankRows = 64, kRankGroups = 32, kRankMax = 262144;
+constexpr uint32_t kRankPad = 1u << 30;  // codes have 30 bits
+
+__global__ __launch_bounds__(256) void rank_tiles(dy_body_view bv, dy_aabb bd, uint32_t n, uint32_t *__restrict__ code,
+                                                  uint32_t *__restrict__ idx, uint64_t *__restrict__ morton64) {
+    __shared__ uint4 key4[kRankTile / 4];
+    __shared__ uint32_t part[4][kRankRows];
+    uint32_t *key = reinterpret_cast<uint32_t *>(key4);
+    const uint32_t t = threadIdx.x, lane = lane_id(), wave = t >> 6;
+    const uint32_t base = blockIdx.y * kRankTile, rows = blockIdx.x;  // rows: block of 64 rows of the tile
+    for (uint32_t k = t; k < kRankTile; k += 256u) {
+        const uint32_t i = base + k;
+        uint32_t code_i = kRankPad + k;  // past the end: behind every code, in order
+        if (i < n) {
+            const uint32_t qx = quantize10(bv.pos_x[i], bd.min_x, bd.max_x);
+            const uint32_t qy = quantize10(bv.pos_y[i], bd.min_y, bd.max_y);
+            const uint32_t qz = quantize10(bv.pos_z[i], bd.min_z, bd.max_z);
+            code_i = morton3(qx, qy, qz);
+        }
+        key[k] = code_i;
+    }
+    __syncthreads();
+    const uint32_t mine = key[rows * kRankRows + lane];
+    uint32_t count = 0;
+    for (uint32_t b = wave * 4u; b < wave * 4u + 4u; ++b) {  // blocks of 64 columns
+        if (b == rows) {
+#pragma unroll 8
+            for (uint32_t c = 0; c < 64u; ++c) {
+                const uint32_t v = key[b * 64u + c];
+                count += v < mine + (c < lane ? 1u : 0u) ? 1u : 0u;
+            }
+        } else {
+            const uint32_t top = mine + (b < rows ? 1u : 0u);  // keys of earlier bodies count when equal
+#pragma unroll
+            for (uint32_t c = 0; c < 16u; ++c) {
+                const uint4 v = key4[b * 16u + c];
+                count += (v.x < top ? 1u : 0u) + (v.y < top ? 1u : 0u) + (v.z < top ? 1u : 0u) + (v.w < top ? 1u : 0u);
+            }
+        }
+    }
+    part[wave][lane] = count;
+    __syncthreads();
+    if (t < kRankRows) {
+        const uint32_t rank = base + part[0][t] + part[1][t] + part[2][t] + part[3][t];
+        const uint32_t i = base + rows * kRankRows + t;
+        code[rank] = mine;
+        idx[rank] = i;
+        if (morton64 && i < n) morton64[rank] = (static_cast<uint64_t>(mine) << 32) | i;
+    }
+}
+
+__global__ __launch_bounds__(kRankTile) void rank_merge(const uint32_t *__restrict__ code, uint32_t n_tiles,
+                                                        uint32_t groups, uint16_t *__restrict__ part) {
+    __shared__ uint32_t key[kRankTile];
+    const uint32_t t = threadIdx.x, row = blockIdx.x, g = blockIdx.y;
+    const uint32_t c0 = static_cast<uint32_t>(static_cast<uint64_t>(g) * n_tiles / groups);
+    const uint32_t c1 = static_cast<uint32_t>(static_cast<uint64_t>(g + 1u) * n_tiles / groups);
+    const uint32_t mine = code[row * kRankTile + t];
+    uint32_t count = 0;
+    for (uint32_t c = c0; c < c1; ++c) {
+        if (c == row) continue;
+        __syncthreads();
+        key[t] = code[c * kRankTile + t];
+        __syncthreads();
+        const uint32_t top = mine + (c < row ? 1u : 0u);
+        uint32_t at = 0;
+#pragma unroll
+        for (uint32_t step = kRankTile / 2u; step > 0u; step >>= 1) at += key[at + step - 1u] < top ? step : 0u;
+        count += at + (key[at] < top ? 1u : 0u);
+    }
+    part[(static_cast<size_t>(g) * n_tiles + row) * kRankTile + t] = static_cast<uint16_t>(count);
+}
+
+__global__ __launch_bounds__(256) void rank_scatter(const uint32_t *__restrict__ code, const uint32_t *__restrict__ idx,
+                                                    const uint16_t *__restrict__ part, uint32_t n, uint32_t n_tiles,
+                                                    uint32_t groups, uint32_t *__restrict__ out_idx,
+                                                    uint64_t *__restrict__ morton64) {
+    const uint32_t p = blockIdx.x * 256u + threadIdx.x;
+    if (p >= n_tiles * kRankTile) return;
+    const uint32_t i = idx[p];
+    uint32_t rank = p % kRankTile;
+#pragma unroll 8
+    for (uint32_t g = 0; g < groups; ++g) rank += part[static_cast<size_t>(g) * n_tiles * kRankTile + p];
+    if (i >= n) return;
+    out_idx[rank] = i;
+    morton64[rank] = (static_cast<uint64_t>(code[p]) << 32) | i;
 }
 
 // ---------------------------------------------------------------------------
@@ -990,6 +1097,7 @@ struct dy_broadphase_s {
     uint32_t *counts = nullptr, *offs = nullptr, *row = nullptr, *ovf = nullptr, *leaf_of = nullptr;
     uint32_t *scan_tmp = nullptr;
     uint32_t *sort_hist = nullptr;  // morton_sort_grid's digit counts, 256 per tile
+    uint16_t *rank_part = nullptr;
     dy_contact_pair *pairs = nullptr;
     uint32_t *count = nullptr;  // = counters + 3
     uint32_t sort_blocks = 0;   // participants of morton_sort_grid per launch (0: single-workgroup sort)
@@ -1016,7 +1124,7 @@ void bp_free(dy_broadphase_s *b) {
     void *ptrs[] = {b->code0, b->idx0, b->code1, b->idx1, b->morton64, b->left, b->right, b->parent,
                     b->root, b->range, b->nodebox, b->tn, b->tp, b->cnt_top, b->entries, b->counters,
                     b->counts, b->offs, b->row, b->ovf, b->leaf_of, b->scan_tmp, b->pairs,
-                    b->sort_hist, b->top_slot, b->top_list};
+                    b->sort_hist, b->rank_part, b->top_slot, b->top_list};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (hipEvent_t &e : b->ev)
@@ -1059,7 +1167,11 @@ int dy_broadphase_create(dy_stream_t s, uint32_t max_bodies, uint32_t max_pairs,
     hipError_t e = hipSuccess;
 #define DY_A(ptr, cnt) \
     if (e == hipSuccess) e = dalloc(ptr, cnt)
-    DY_A(b->code0, nb); DY_A(b->idx0, nb); DY_A(b->code1, nb); DY_A(b->idx1, nb);
+    // rank_tiles writes whole tiles; rank_merge has a count per key and group of tiles
+    const size_t padded = (nb + kRankTile - 1) / kRankTile * kRankTile;
+    const size_t ranked = padded < kRankMax ? padded : kRankMax;
+    DY_A(b->code0, padded); DY_A(b->idx0, padded); DY_A(b->code1, padded); DY_A(b->idx1, padded);
+    DY_A(b->rank_part, ranked * (ranked / kRankTile < kRankGroups ? ranked / kRankTile : kRankGroups));
     DY_A(b->morton64, nb);
     DY_A(b->left, nb); DY_A(b->right, nb); DY_A(b->parent, nodes); DY_A(b->root, 1);
     DY_A(b->range, nb); DY_A(b->nodebox, nodes); DY_A(b->tn, nodes); DY_A(b->tp, nb);
@@ -1136,7 +1248,24 @@ int dy_broadphase_build_and_query(dy_broadphase_t bp, dy_stream_t s, const dy_bo
     const int ni = static_cast<int>(n);
     const uint32_t n_tiles = ceil_div(n, kSgTile);
     bool sorted = false;
-    if (bp->sort_blocks > 0 && n_tiles > 4) {
+    if (!bp->sort_fixed && n <= kRankMax) {
+        const uint32_t tiles = ceil_div(n, kRankTile);
+        if (tiles == 1) {
+            rank_tiles<<<dim3(ceil_div(n, kRankRows), 1), 256, 0, st>>>(*bodies, *bounds, n, bp->code0, bp->idx0,
+                                                                         bp->morton64);
+        } else {
+            const uint32_t groups = tiles < kRankGroups ? tiles : kRankGroups;
+            rank_tiles<<<dim3(kRankTile / kRankRows, tiles), 256, 0, st>>>(*bodies, *bounds, n, bp->code1, bp->idx1,
+                                                                            nullptr);
+            DY_LAUNCH_CHECK();
+            rank_merge<<<dim3(tiles, groups), kRankTile, 0, st>>>(bp->code1, tiles, groups, bp->rank_part);
+            DY_LAUNCH_CHECK();
+            rank_scatter<<<ceil_div(tiles * kRankTile, 256), 256, 0, st>>>(bp->code1, bp->idx1, bp->rank_part, n, tiles,
+                                                                            groups, bp->idx0, bp->morton64);
+        }
+        DY_LAUNCH_CHECK();
+        sorted = true;
+    } else if (bp->sort_blocks > 0 && n_tiles > 4) {
         // sort_blocks participants on one XCD out of a launch with as many on
         // every XCD (8 on gfx950)
         // one participant per tile (each sorts one tile per pass), fewer when
