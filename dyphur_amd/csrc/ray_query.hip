@@ -140,7 +140,7 @@ __device__ __forceinline__ bool rq_box(const uint4 &nb, const float o[3], const 
 }
 
 // One ray's walk as the reference does it, by one lane, from the view's arrays.
-__device__ __noinline__ dy_ray_hit rq_walk(const dy_bvh_view &bvh, const dy_body_view &bv, const dy_shape_view &sv,
+__device__ __forceinline__ dy_ray_hit rq_walk(const dy_bvh_view &bvh, const dy_body_view &bv, const dy_shape_view &sv,
                                            const dy_ray &r) {
     const float o[3] = {r.ox, r.oy, r.oz}, d[3] = {r.dx, r.dy, r.dz};
     const float inv[3] = {1.f / r.dx, 1.f / r.dy, 1.f / r.dz};
@@ -166,6 +166,20 @@ __device__ __noinline__ dy_ray_hit rq_walk(const dy_bvh_view &bvh, const dy_body
         }
     }
     return hit;
+}
+
+// The same out of line, for the rays that a team gives up.
+__device__ __noinline__ dy_ray_hit rq_walk_apart(const dy_bvh_view &bvh, const dy_body_view &bv,
+                                                 const dy_shape_view &sv, const dy_ray &r) {
+    return rq_walk(bvh, bv, sv, r);
+}
+
+// One ray a lane: the form for many rays over few bodies (see ray_lanes).
+__global__ __launch_bounds__(256) void ray_query_lanes(dy_bvh_view bvh, dy_body_view bv, dy_shape_view sv,
+                                                       const dy_ray *__restrict__ rays, dy_ray_hit *__restrict__ hits,
+                                                       uint32_t n_rays) {
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n_rays) hits[k] = rq_walk(bvh, bv, sv, rays[k]);
 }
 
 // A team of kRqTeam lanes walks one ray.  The reference's result is a fold over
@@ -482,7 +496,22 @@ __global__ __launch_bounds__(64) void ray_query_kernel(dy_bvh_view bvh, dy_body_
             next = least + 1u;
         }
     }
-    if (mine && tl == 0) hits[k] = odd ? rq_walk(bvh, bv, sv, r) : dy_ray_hit{best, best_body};
+    if (mine && tl == 0) hits[k] = odd ? rq_walk_apart(bvh, bv, sv, r) : dy_ray_hit{best, best_body};
+}
+
+// One lane a ray (ray_query_lanes) or a team?  The lanes take as long as the
+// longest walk however few the rays (20 us over 10 bodies, 300 over 1 000), and
+// beyond a full chip 0.05 ns a ray over 10 bodies and 3 over 30 000; teams start
+// at a tenth of that, and take 0.9 to 2.8 ns.  So many rays over few bodies are
+// the lanes'.  Teams / lanes over a pile: 10 bodies 3 000 rays 16 / 19 us, 10 000
+// rays 29 / 20; 100 bodies 30 000 rays 60 / 75, 200 000 rays 254 / 94; 1 000 bodies
+// 100 000 rays 195 / 308, 200 000 rays 353 / 313; 8 000 bodies 400 000 rays
+// 916 / 973, 800 000 rays 1 754 / 1 508; 30 000 bodies 2 000 000 rays 5 680 / 6 530.
+// The lines follow the counts at which both took the same time.
+static bool ray_lanes(uint32_t n, uint32_t n_rays) {
+    const uint64_t m = n_rays;
+    if (n <= 4u || m >= 550ull * n) return true;
+    return n <= 16384u && m >= 60ull * n && m * m >= 5400ull * 5400ull * n;
 }
 
 }  // namespace dy
@@ -496,7 +525,13 @@ int dy_ray_query(dy_stream_t s, const dy_bvh_view *bvh, const dy_body_view *bodi
     if (!bvh || !bodies || !shapes || (n_rays && (!d_rays || !d_hits))) return DY_ERR_INVALID_ARG;
     if (n_rays == 0) return DY_OK;
     if (bvh->n > bodies->n) return DY_ERR_INVALID_ARG;
-    const uint32_t n = bvh->n, blocks = ceil_div(n_rays, kRqTeams);
+    const uint32_t n = bvh->n;
+    if (ray_lanes(n, n_rays)) {
+        ray_query_lanes<<<ceil_div(n_rays, 256), 256, 0, hs(s)>>>(*bvh, *bodies, *shapes, d_rays, d_hits, n_rays);
+        DY_LAUNCH_CHECK();
+        return DY_OK;
+    }
+    const uint32_t blocks = ceil_div(n_rays, kRqTeams);
     // Records are made for the call where enough rays read them (they cost an
     // allocation and a launch, about 33 us of a small call): 40 000 bodies with
     // 500 rays 117 us with and 112 without, 5 000 rays 153 / 182, 20 000 rays

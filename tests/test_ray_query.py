@@ -5,6 +5,8 @@ CPU: the oracle against the reference's known answers
 bodies (the closest exact hit among bodies whose binary16 leaf box the ray
 enters); GPU: dy_ray_query bit for bit against the oracle.
 """
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -192,6 +194,39 @@ def test_gpu_ray_query_teams_bitexact(gpu, oracle, n, m, moved, axis):
             db.f[f].upload(v, s)
             b.arr[f][:] = v
     t_ref, b_ref = w.ray_query(b, osh, sc.n, rays)
+    t, body = gpu.ray_query(s, bp, sc.n, db, ds, rays)
+    assert np.array_equal(body, b_ref)
+    assert np.array_equal(t.view(np.uint32), t_ref.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m,axis", [(1, 300, False), (4, 700, True), (5, 2749, False), (5, 2750, True),
+                                      (119, 65450, True), (300, 93530, False), (300, 93531, False)])
+def test_gpu_ray_query_lanes_bitexact(gpu, oracle, n, m, axis):
+    """Many rays over few bodies go one a lane: both sides of the lines between
+    lanes and teams, with and without rays along the axes."""
+    rng = np.random.default_rng(n + m)
+    side = 1.2 * n ** (1 / 3) + 1.0
+    sc = scenes.random_mixed(max(n - 1, 1), seed=6, extent=(side, side, side))
+    if n == 1:
+        sc = dataclasses.replace(sc, **{k: getattr(sc, k)[:1] for k in ("pos", "rot", "vel", "ang", "mass", "inertia",
+                                                                        "shape", "flags")})
+    print(f"[ray lanes] n={sc.n} rays={m} axis={axis}", flush=True)
+    o = rng.uniform(-side, side, (m, 3))
+    d = rng.uniform(-side, side, (m, 3)) + [0, side / 2, 0] - o
+    if axis:
+        keep = rng.integers(0, 3, m)
+        d = np.zeros((m, 3))
+        d[np.arange(m), keep] = np.where(rng.random(m) < 0.5, 1.0, -1.0)
+        o[: m // 2] = np.round(o[: m // 2] * 4) / 4
+    t_max = rng.choice([0.5, 3.0, 50.0, np.inf], m)
+    rays = np.hstack([o, d, t_max[:, None]]).astype(F32)
+    (t_ref, b_ref), _, _, _ = _oracle_query(oracle, sc, list(rays))
+    s = gpu.Stream()
+    db = gpu.DeviceBodies(sc, s)
+    ds = gpu.DeviceShapes(sc, s)
+    bp = gpu.Broadphase(s, sc.n, sc.max_pairs)
+    bp.build_and_query(s, db, ds, sc.bounds)
     t, body = gpu.ray_query(s, bp, sc.n, db, ds, rays)
     assert np.array_equal(body, b_ref)
     assert np.array_equal(t.view(np.uint32), t_ref.view(np.uint32))
