@@ -514,6 +514,20 @@ static bool ray_lanes(uint32_t n, uint32_t n_rays) {
     return n <= 16384u && m >= 60ull * n && m * m >= 5400ull * 5400ull * n;
 }
 
+// Rays of one launch: 16 threads each stay below the 2^32 threads that a grid may have.
+constexpr uint32_t kRqLaunch = 1u << 27;
+
+// launch(first, count) for the rays in runs that one grid can take.
+template <class F>
+static int ray_launches(uint32_t n_rays, F &&launch) {
+    for (uint64_t k = 0; k < n_rays; k += kRqLaunch) {
+        const uint64_t left = n_rays - k;
+        launch(static_cast<size_t>(k), static_cast<uint32_t>(left < kRqLaunch ? left : kRqLaunch));
+        DY_LAUNCH_CHECK();
+    }
+    return DY_OK;
+}
+
 }  // namespace dy
 
 using namespace dy;
@@ -526,32 +540,36 @@ int dy_ray_query(dy_stream_t s, const dy_bvh_view *bvh, const dy_body_view *bodi
     if (n_rays == 0) return DY_OK;
     if (bvh->n > bodies->n) return DY_ERR_INVALID_ARG;
     const uint32_t n = bvh->n;
-    if (ray_lanes(n, n_rays)) {
-        ray_query_lanes<<<ceil_div(n_rays, 256), 256, 0, hs(s)>>>(*bvh, *bodies, *shapes, d_rays, d_hits, n_rays);
-        DY_LAUNCH_CHECK();
-        return DY_OK;
-    }
-    const uint32_t blocks = ceil_div(n_rays, kRqTeams);
+    if (ray_lanes(n, n_rays))
+        return ray_launches(n_rays, [&](size_t k, uint32_t m) {
+            ray_query_lanes<<<ceil_div(m, 256), 256, 0, hs(s)>>>(*bvh, *bodies, *shapes, d_rays + k, d_hits + k, m);
+        });
+    const auto teams = [&](const RqRecords *rec) {
+        return ray_launches(n_rays, [&](size_t k, uint32_t m) {
+            const uint32_t blocks = ceil_div(m, kRqTeams);
+            if (rec)
+                ray_query_kernel<true><<<blocks, 64, 0, hs(s)>>>(*bvh, *bodies, *shapes, *rec, d_rays + k, d_hits + k, m);
+            else
+                ray_query_kernel<false><<<blocks, 64, 0, hs(s)>>>(*bvh, *bodies, *shapes, RqRecords{}, d_rays + k,
+                                                                  d_hits + k, m);
+        });
+    };
     // Records are made for the call where enough rays read them (they cost an
     // allocation and a launch, about 33 us of a small call): 40 000 bodies with
     // 500 rays 117 us with and 112 without, 5 000 rays 153 / 182, 20 000 rays
     // 203 / 263; 1 000 bodies with 500 rays 67 / 34, 20 000 rays 73 / 83.  Not
     // under capture, where nothing is allocated.
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (n_rays >= 4096u && n_rays >= n / 16u && n > 1u) DY_TRY(hipStreamIsCapturing(hs(s), &capture));
-    if (n_rays < 4096u || n_rays < n / 16u || n < 2u || capture != hipStreamCaptureStatusNone) {
-        ray_query_kernel<false><<<blocks, 64, 0, hs(s)>>>(*bvh, *bodies, *shapes, RqRecords{}, d_rays, d_hits, n_rays);
-        DY_LAUNCH_CHECK();
-        return DY_OK;
-    }
+    const bool many = n_rays >= 4096u && n_rays >= n / 16u;
+    if (many) DY_TRY(hipStreamIsCapturing(hs(s), &capture));
+    if (!many || capture != hipStreamCaptureStatusNone) return teams(nullptr);
     uint4 *p = nullptr;
     DY_TRY(hipMallocAsync(reinterpret_cast<void **>(&p), 5 * static_cast<size_t>(n) * sizeof(uint4), hs(s)));
     const RqRecords rec{p, reinterpret_cast<float4 *>(p + 2 * static_cast<size_t>(n))};
     ray_records<<<ceil_div(n, 256), 256, 0, hs(s)>>>(*bvh, *bodies, *shapes, rec);
-    ray_query_kernel<true><<<blocks, 64, 0, hs(s)>>>(*bvh, *bodies, *shapes, rec, d_rays, d_hits, n_rays);
-    const hipError_t launched = hipGetLastError();
+    const int st = teams(&rec);
     DY_TRY(hipFreeAsync(p, hs(s)));
-    return static_cast<int>(launched);
+    return st;
 }
 
 }  // extern "C"

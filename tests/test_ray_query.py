@@ -230,3 +230,46 @@ def test_gpu_ray_query_lanes_bitexact(gpu, oracle, n, m, axis):
     t, body = gpu.ray_query(s, bp, sc.n, db, ds, rays)
     assert np.array_equal(body, b_ref)
     assert np.array_equal(t.view(np.uint32), t_ref.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m", [(20000, 2**28 + 5), (40, 2**27 + 3)])
+def test_gpu_ray_query_more_rays_than_one_grid(gpu, n, m):
+    """More rays than one launch's grid can take (teams from 2^28 rays on, and
+    the first run's end among the lanes): every ray has its own hit."""
+    import ctypes
+    side = 1.2 * n ** (1 / 3)
+    sc = scenes.random_mixed(n - 1, seed=5, extent=(side, side, side))
+    print(f"[rays past one grid] n={sc.n} rays={m}", flush=True)
+    s = gpu.Stream()
+    db, ds = gpu.DeviceBodies(sc, s), gpu.DeviceShapes(sc, s)
+    bp = gpu.Broadphase(s, sc.n, sc.max_pairs)
+    bp.build_and_query(s, db, ds, sc.bounds)
+    rng = np.random.default_rng(2)
+    some = 4093
+    o = rng.uniform(-side, side, (some, 3))
+    d = rng.uniform(-side, side, (some, 3)) - o
+    few = np.hstack([o, d, np.full((some, 1), 2.0)]).astype(F32)
+    t, body = gpu.ray_query(s, bp, sc.n, db, ds, few)
+    want = np.stack([t.view(np.uint32), body], 1)
+    rays = gpu.DeviceArray(7 * m, F32)
+    rays.upload(few.ravel(), s, 7 * some)
+    have = some
+    while have < m:  # the same rays again and again
+        more = min(have, m - have)
+        gpu.check(gpu.lib().dy_memcpy_d2d_async(gpu.vp(rays.ptr + 28 * have), gpu.vp(rays.ptr), 28 * more, s.h), "copy")
+        have += more
+    hits = gpu.DeviceArray(2 * m, np.uint32)
+    bvh = gpu.BvhView()
+    gpu.check(gpu.lib().dy_broadphase_bvh_view(bp.h, sc.n, ctypes.byref(bvh)), "view")
+    bv, sv = db.view(), ds.view()
+    gpu.check(gpu.lib().dy_ray_query(s.h, ctypes.byref(bvh), ctypes.byref(bv), ctypes.byref(sv), rays.ptr, hits.ptr, m),
+              "dy_ray_query")
+    for k in range(0, m, 4096 * some):
+        part = min(4096 * some, m - k)
+        got = gpu.download_ptr(hits.ptr + 8 * k, 2 * part, np.uint32, s).reshape(part, 2)
+        whole = part // some * some
+        assert np.all(got[:whole].reshape(-1, some, 2) == want), k
+        assert np.array_equal(got[whole:], want[: part - whole]), k
+    rays.free()
+    hits.free()
