@@ -558,13 +558,16 @@ int dy_ray_query(dy_stream_t s, const dy_bvh_view *bvh, const dy_body_view *bodi
     // allocation and a launch, about 33 us of a small call): 40 000 bodies with
     // 500 rays 117 us with and 112 without, 5 000 rays 153 / 182, 20 000 rays
     // 203 / 263; 1 000 bodies with 500 rays 67 / 34, 20 000 rays 73 / 83.  Not
-    // under capture, where nothing is allocated.
+    // under capture, where nothing is allocated, nor where memory is short.
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     const bool many = n_rays >= 4096u && n_rays >= n / 16u;
     if (many) DY_TRY(hipStreamIsCapturing(hs(s), &capture));
     if (!many || capture != hipStreamCaptureStatusNone) return teams(nullptr);
     uint4 *p = nullptr;
-    DY_TRY(hipMallocAsync(reinterpret_cast<void **>(&p), 5 * static_cast<size_t>(n) * sizeof(uint4), hs(s)));
+    if (hipMallocAsync(reinterpret_cast<void **>(&p), 5 * static_cast<size_t>(n) * sizeof(uint4), hs(s)) != hipSuccess) {
+        (void)hipGetLastError();  // no room: the view's arrays will do
+        return teams(nullptr);
+    }
     const RqRecords rec{p, reinterpret_cast<float4 *>(p + 2 * static_cast<size_t>(n))};
     ray_records<<<ceil_div(n, 256), 256, 0, hs(s)>>>(*bvh, *bodies, *shapes, rec);
     const int st = teams(&rec);

@@ -5,6 +5,7 @@ CPU: the oracle against the reference's known answers
 bodies (the closest exact hit among bodies whose binary16 leaf box the ray
 enters); GPU: dy_ray_query bit for bit against the oracle.
 """
+import ctypes
 import dataclasses
 
 import numpy as np
@@ -237,7 +238,6 @@ def test_gpu_ray_query_lanes_bitexact(gpu, oracle, n, m, axis):
 def test_gpu_ray_query_more_rays_than_one_grid(gpu, n, m):
     """More rays than one launch's grid can take (teams from 2^28 rays on, and
     the first run's end among the lanes): every ray has its own hit."""
-    import ctypes
     side = 1.2 * n ** (1 / 3)
     sc = scenes.random_mixed(n - 1, seed=5, extent=(side, side, side))
     print(f"[rays past one grid] n={sc.n} rays={m}", flush=True)
@@ -273,3 +273,61 @@ def test_gpu_ray_query_more_rays_than_one_grid(gpu, n, m):
         assert np.array_equal(got[whole:], want[: part - whole]), k
     rays.free()
     hits.free()
+
+
+class _SmallPool:
+    """The device's stream-ordered allocations from a pool of at most `size`
+    bytes while it is open."""
+
+    class Props(ctypes.Structure):  # hipMemPoolProps
+        _fields_ = [("alloc_type", ctypes.c_int), ("handle_types", ctypes.c_int), ("location_type", ctypes.c_int),
+                    ("location_id", ctypes.c_int), ("security", ctypes.c_void_p), ("max_size", ctypes.c_size_t),
+                    ("reserved", ctypes.c_ubyte * 56)]
+
+    def __init__(self, hip, size):
+        self.hip = hip  # a library that the runtime's own entry points are found through
+        self.size, self.pool, self.old = size, ctypes.c_void_p(), ctypes.c_void_p()
+
+    def __enter__(self):
+        p = self.Props(alloc_type=1, location_type=1, max_size=self.size)
+        assert self.hip.hipDeviceGetMemPool(ctypes.byref(self.old), 0) == 0
+        assert self.hip.hipMemPoolCreate(ctypes.byref(self.pool), ctypes.byref(p)) == 0
+        assert self.hip.hipDeviceSetMemPool(0, self.pool) == 0
+        return self
+
+    def take(self, size, s):
+        """What an allocation of `size` bytes on stream s returns."""
+        q = ctypes.c_void_p()
+        st = self.hip.hipMallocAsync(ctypes.byref(q), ctypes.c_size_t(size), s.h)
+        if st == 0:
+            assert self.hip.hipFreeAsync(q, s.h) == 0
+        self.hip.hipGetLastError()
+        return st
+
+    def __exit__(self, *exc):
+        assert self.hip.hipDeviceSetMemPool(0, self.old) == 0
+        assert self.hip.hipDeviceSynchronize() == 0
+        assert self.hip.hipMemPoolDestroy(self.pool) == 0
+
+
+@pytest.mark.gpu
+def test_gpu_ray_query_without_room_for_records(gpu, oracle):
+    """A call whose scratch allocation fails walks the view's arrays instead."""
+    n, m = 20000, 5000
+    side = 1.2 * n ** (1 / 3)
+    sc = scenes.random_mixed(n - 1, seed=5, extent=(side, side, side))
+    print(f"[rays without records] n={sc.n} rays={m}", flush=True)
+    rng = np.random.default_rng(4)
+    o = rng.uniform(-side, side, (m, 3))
+    rays = np.hstack([o, rng.uniform(-side, side, (m, 3)) - o, np.full((m, 1), 2.0)]).astype(F32)
+    (t_ref, b_ref), *_ = _oracle_query(oracle, sc, list(rays))
+    s = gpu.Stream()
+    db, ds = gpu.DeviceBodies(sc, s), gpu.DeviceShapes(sc, s)
+    bp = gpu.Broadphase(s, sc.n, sc.max_pairs)
+    bp.build_and_query(s, db, ds, sc.bounds)
+    s.wait()
+    with _SmallPool(gpu.lib(), 1 << 16) as pool:
+        assert pool.take(80 * n, s) != 0
+        t, body = gpu.ray_query(s, bp, sc.n, db, ds, rays)
+    assert np.array_equal(body, b_ref)
+    assert np.array_equal(t.view(np.uint32), t_ref.view(np.uint32))
