@@ -275,6 +275,72 @@ def test_gpu_ray_query_more_rays_than_one_grid(gpu, n, m):
     hits.free()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m", [(200, 4000), (2000, 20000), (4, 4000)])
+def test_gpu_ray_query_not_finite(gpu, oracle, n, m):
+    """Directions, origins and t_max that are infinite, zero or no number, and
+    bodies whose binary16 boxes are infinite: teams from the view's arrays and
+    from records, and lanes."""
+    rng = np.random.default_rng(n + m)
+    side = 1.2 * n ** (1 / 3) + 1.0
+    sc = scenes.random_mixed(n - 1, seed=8, extent=(side, side, side))
+    sc.pos[::3, 0] += F32(1e5)  # past 65 504
+    sc.pos[1::7, 1] -= F32(2e5)
+    print(f"[ray not finite] n={sc.n} rays={m}", flush=True)
+    o = rng.uniform(-side, side, (m, 3))
+    target = sc.pos[rng.integers(0, sc.n, m)].astype(np.float64)
+    d = (target - o) * rng.choice([1.0, 1e-3], (m, 1))
+    odd = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 1e-40, 3e38])
+    pick = rng.random((m, 3)) < 0.35
+    d = np.where(pick, odd[rng.integers(0, len(odd), (m, 3))], d)
+    far = np.array([np.inf, -np.inf, np.nan, 1e5, 3.4e38, 0.0])
+    pick = rng.random((m, 3)) < 0.05
+    o = np.where(pick, far[rng.integers(0, len(far), (m, 3))], o)
+    t_max = rng.choice([0.0, -1.0, 1.0, 50.0, 3e38, np.inf, -np.inf, np.nan], m, p=[.05, .05, .1, .2, .2, .3, .05, .05])
+    rays = np.hstack([o, d, t_max[:, None]]).astype(F32)
+    (t_ref, b_ref), *_ = _oracle_query(oracle, sc, list(rays))
+    s = gpu.Stream()
+    db, ds = gpu.DeviceBodies(sc, s), gpu.DeviceShapes(sc, s)
+    bp = gpu.Broadphase(s, sc.n, sc.max_pairs)
+    bp.build_and_query(s, db, ds, sc.bounds)
+    t, body = gpu.ray_query(s, bp, sc.n, db, ds, rays)
+    assert np.array_equal(body, b_ref)
+    same = t.view(np.uint32) == t_ref.view(np.uint32)
+    assert np.all(same | (np.isnan(t) & np.isnan(t_ref)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m", [(2000, 5000), (90, 60000)])
+def test_gpu_ray_query_captured(gpu, n, m):
+    """A captured query (teams without records, lanes) replays to the eager
+    result, with eager work and moved bodies between the replays."""
+    rng = np.random.default_rng(n)
+    side = 1.2 * n ** (1 / 3)
+    sc = scenes.random_mixed(n - 1, seed=9, extent=(side, side, side))
+    print(f"[ray captured] n={sc.n} rays={m}", flush=True)
+    o = rng.uniform(-side, side, (m, 3))
+    rays = np.hstack([o, rng.uniform(-side, side, (m, 3)) - o, np.full((m, 1), 3.0)]).astype(F32)
+    s = gpu.Stream()
+    db, ds = gpu.DeviceBodies(sc, s), gpu.DeviceShapes(sc, s)
+    bp = gpu.Broadphase(s, sc.n, sc.max_pairs)
+    bp.build_and_query(s, db, ds, sc.bounds)
+    d_rays = gpu.DeviceArray.from_numpy(rays.ravel(), s)
+    d_hits = gpu.DeviceArray(2 * m, np.uint32)
+    bvh = gpu.BvhView()
+    gpu.check(gpu.lib().dy_broadphase_bvh_view(bp.h, sc.n, ctypes.byref(bvh)), "view")
+    bv, sv = db.view(), ds.view()
+    with gpu.Graph.capture(s) as g:
+        gpu.check(gpu.lib().dy_ray_query(s.h, ctypes.byref(bvh), ctypes.byref(bv), ctypes.byref(sv), d_rays.ptr,
+                                         d_hits.ptr, m), "dy_ray_query")
+    for _ in range(4):
+        db.f["pos_x"].upload(sc.pos[:, 0] + rng.uniform(-0.2, 0.2, sc.n).astype(F32), s)
+        t, body = gpu.ray_query(s, bp, sc.n, db, ds, rays)
+        d_hits.upload(np.zeros(2 * m, np.uint32), s)
+        g.launch(s)
+        got = d_hits.download(s).reshape(m, 2)
+        assert np.array_equal(got[:, 1], body) and np.array_equal(got[:, 0], t.view(np.uint32))
+
+
 class _SmallPool:
     """The device's stream-ordered allocations from a pool of at most `size`
     bytes while it is open."""
