@@ -1801,6 +1801,7 @@ struct dy_xpbd_s {
     int assign_threads = 256, sweep_threads = 256;
     int path = 0;  // 0 cooperative kernels, 1 one launch per round / per class
     bool coop_refused = false;  // a cooperative launch was refused: launches per round / per class from now on
+    int refuse = 0;  // launches to take as refused (DYPHUR_REFUSE_LAUNCH): 1 assignment, 2 motors, 4 sweep_first, 8 sweeps
     // Kernel timing (dy_xpbd_set_timing): event pairs recorded around the
     // assignment and sweep kernels, read back once the next solve syncs.
     bool timing = false;
@@ -1943,7 +1944,8 @@ int env_int(const char *name, int dflt) {
 // phases over the whole grid), DYPHUR_SWEEP_PAIR (0: contact-only dataflow
 // sweeps with one lane per record instead of a pair), DYPHUR_SWEEP_PAIR_THREADS
 // and DYPHUR_SOLVER_PATH (1 = one launch per round / per class) override the
-// launch shapes for measurement.
+// launch shapes for measurement; DYPHUR_REFUSE_LAUNCH takes launches as refused
+// (see dy_xpbd_s::refuse) so that what follows a refusal can be tested.
 int query_coop(dy_xpbd_s *x) {
     int dev = 0, coop = 0;
     DY_TRY(hipGetDevice(&dev));
@@ -1952,6 +1954,7 @@ int query_coop(dy_xpbd_s *x) {
     x->sweep_blocks_override = env_int("DYPHUR_SWEEP_BLOCKS", 0);
     x->assign_blocks_override = env_int("DYPHUR_ASSIGN_BLOCKS", 0);
     x->path = env_int("DYPHUR_SOLVER_PATH", 0);
+    x->refuse = env_int("DYPHUR_REFUSE_LAUNCH", 0);
     {
         const int m = env_int("DYPHUR_SWEEP_MODE", 2);
         x->sweep_mode = (m == 0 || m == 1 || m == 3) ? m : 2;
@@ -2005,6 +2008,13 @@ uint32_t coop_blocks(const dy_xpbd_s *x, int override_blocks, int threads, int m
     if (b < 1) b = 1;
     if (b > max_blocks) b = max_blocks;
     return static_cast<uint32_t>(b);
+}
+
+// try_coop_launch of one of the solver's kernels (`kind`: its bit in x->refuse); false when refused.
+bool grid_launch(const dy_xpbd_s *x, int kind, const void *fn, uint32_t blocks, int threads, void **args,
+                 hipStream_t st) {
+    return !(x->refuse & kind) &&
+           try_coop_launch(fn, dim3(blocks), dim3(static_cast<uint32_t>(threads)), args, st) == hipSuccess;
 }
 
 // Launch-per-round assignment: the host drives the rounds and decides the
@@ -2181,9 +2191,10 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
                                                         : ceil_div(nb ? nb : 1u, static_cast<uint32_t>(x->assign_threads));
         if (one_xcd) blocks *= 8u;  // an eighth of a launch runs on the XCD
         if (blocks > most) blocks = most;
-        if (try_coop_launch(one_xcd ? reinterpret_cast<const void *>(assign_flow<true>)
-                                    : reinterpret_cast<const void *>(assign_flow<false>),
-                            dim3(blocks), dim3(static_cast<uint32_t>(x->assign_threads)), args, st) != hipSuccess) {
+        if (!grid_launch(x, 1,
+                         one_xcd ? reinterpret_cast<const void *>(assign_flow<true>)
+                                 : reinterpret_cast<const void *>(assign_flow<false>),
+                         blocks, x->assign_threads, args, st)) {
             x->coop_refused = true;
             coop = false;
         }
@@ -2216,8 +2227,7 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
             float dtv = dt;
             uint32_t *metav = x->meta;
             void *args[] = {&boffv, &rec, &dynv, &stav, &jpkv0, &dtv, &metav};
-            motors = try_coop_launch(reinterpret_cast<const void *>(joint_motors_xcd), dim3(blocks),
-                                     dim3(static_cast<uint32_t>(x->sweep_threads)), args, st) == hipSuccess;
+            motors = grid_launch(x, 2, reinterpret_cast<const void *>(joint_motors_xcd), blocks, x->sweep_threads, args, st);
             if (!motors) {
                 x->coop_refused = true;
                 coop = false;
@@ -2250,18 +2260,21 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
         float muv = x->mu, dtv = dt;
         uint32_t *metav = x->meta;
         void *args[] = {&rec, &rseqv, &lamv, &bwv, &stav, &muv, &dtv, &metav};
-        if (try_coop_launch(one_xcd ? reinterpret_cast<const void *>(sweep_first<true>)
-                                    : reinterpret_cast<const void *>(sweep_first<false>),
-                            dim3(blocks), dim3(static_cast<uint32_t>(x->pair_threads)), args, st) != hipSuccess) {
+        if (!grid_launch(x, 4,
+                         one_xcd ? reinterpret_cast<const void *>(sweep_first<true>)
+                                 : reinterpret_cast<const void *>(sweep_first<false>),
+                         blocks, x->pair_threads, args, st)) {
             x->coop_refused = true;
             coop = false;
             words = false;
         }
     }
-    if (gathered && !words) {
+    const auto to_records = [&]() -> int {
         words_to_records<<<ceil_div(nb ? nb : 1u, 256), 256, 0, st>>>(x->bw.p, nb, x->dyn.p);
         DY_LAUNCH_CHECK();
-    }
+        return DY_OK;
+    };
+    if (gathered && !words) DY_TRY_STATUS(to_records());
     if (words && iters == 1u) swept = true;
     if (!swept && coop && flow) {
         // one workgroup of pair_threads per CU of the XCD by default (the
@@ -2293,7 +2306,7 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
             fn = reinterpret_cast<const void *>(sweep_flow_pair);
         else
             fn = J ? reinterpret_cast<const void *>(sweep_flow<true>) : reinterpret_cast<const void *>(sweep_flow<false>);
-        swept = try_coop_launch(fn, dim3(blocks), dim3(static_cast<uint32_t>(threads)), args, st) == hipSuccess;
+        swept = grid_launch(x, 8, fn, blocks, threads, args, st);
     } else if (!swept && coop) {
         // sweep_xcd: P participants on one XCD out of a launch of P per XCD
         // (8 XCDs on gfx950); sweep_persistent: P workgroups over the chip.
@@ -2317,16 +2330,20 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
         else
             fn = J ? reinterpret_cast<const void *>(sweep_persistent<true>)
                    : reinterpret_cast<const void *>(sweep_persistent<false>);
-        swept = try_coop_launch(fn, dim3(blocks), dim3(static_cast<uint32_t>(x->sweep_threads)), args, st) == hipSuccess;
+        swept = grid_launch(x, 8, fn, blocks, x->sweep_threads, args, st);
     }
     if (!swept) {
         if (coop) x->coop_refused = true;
-        // Per-class launches; the class count is read back first.
+        // Per-class launches; the class count is read back first.  Where
+        // sweep_first has run, they go on after it, from the words it left.
         uint32_t k = 0;
+        const uint32_t first = words ? 1u : 0u;
+        if (words) DY_TRY_STATUS(to_records());
+        words = false;
         DY_TRY(hipMemcpyAsync(&k, x->meta + kMNcls, sizeof(k), hipMemcpyDeviceToHost, st));
         DY_TRY(hipStreamSynchronize(st));
         const uint32_t blocks = grid_for(ncap);
-        for (uint32_t it = 0; it < iters; ++it)
+        for (uint32_t it = first; it < iters; ++it)
             for (uint32_t c = 0; c < k; ++c) {
                 if (J)
                     sweep_class<true><<<blocks, kSolveThreads, 0, st>>>(x->boff, c, it, rec, x->lam, x->dyn.p,

@@ -126,3 +126,57 @@ def test_first_iteration_by_words_matches_records(gpu, monkeypatch, n, nc, iters
         got.append(db.download(s))
     for k in got[0]:
         assert np.array_equal(np.asarray(got[0][k]).view(np.uint32), np.asarray(got[1][k]).view(np.uint32)), k
+
+
+def _plates(n):
+    """n - 1 dynamic bodies over one static one, six contacts each with it, that
+    stay live after the first iteration: their inertia about z and their mass
+    are so large that a contact which pushes along their plane (a third of them)
+    cannot move them until another one has turned the plane."""
+    rng = np.random.default_rng(n)
+    sc = scenes.random_mixed(n - 1, seed=2, extent=(40, 40, 40))
+    sc.mass = np.where(np.arange(n) < n - 1, 1e13, 0.0).astype(np.float32)
+    sc.flags = np.where(np.arange(n) < n - 1, 0, scenes.FLAG_STATIC).astype(np.uint32)
+    sc.rot[:] = 1.0, 0.0, 0.0, 0.0
+    sc.inertia[:] = 0.0
+    sc.inertia[:, [0, 4, 8]] = 1.0, 1.0, 1e13
+    a = np.repeat(np.arange(n - 1), 6)
+    nc = len(a)
+    b = np.full(nc, n - 1)
+    turn = rng.random(nc) < 2 / 3
+    angle = rng.uniform(0, 2 * np.pi, nc)
+    normal = np.where(turn, [[0.0]] * 2 + [[1.0]], [np.cos(angle), np.sin(angle), 0.0 * angle])
+    arm = rng.uniform(0.2, 0.5, (3, nc)) * [[1], [1], [0]]
+    return sc, a, b, [v.astype(np.float32) for v in (*(sc.pos[a].T + arm), *normal, rng.uniform(0.01, 0.05, nc))]
+
+
+def _solved(gpu, sc, a, b, fields, iters, solves=1):
+    s = gpu.Stream()
+    db = gpu.DeviceBodies(sc, s)
+    solver = gpu.XpbdSolver(s, iters, len(a), 0.5)
+    cv, _keep = _view(gpu, s, a.astype(np.uint32), b.astype(np.uint32), fields)
+    for _ in range(solves):
+        solver.solve(s, cv, db, sc.dt)
+    assert solver.stats()["n_constraints"] == len(a)
+    return db.download(s)
+
+
+def _same_bits(x, y):
+    return all(np.array_equal(np.asarray(x[k]).view(np.uint32), np.asarray(y[k]).view(np.uint32)) for k in x)
+
+
+@pytest.mark.parametrize("n", [60, 3000, 16400])
+@pytest.mark.parametrize("refuse", [1, 4, 8])
+def test_refused_launches_change_nothing(gpu, monkeypatch, n, refuse):
+    """A refused launch of the assignment (1), the first iteration (4) or the
+    later ones (8), in the solve that meets it and in the next one, with
+    contacts that only the later iterations move."""
+    print(f"[refused] n={n} refuse={refuse}", flush=True)
+    sc, a, b, fields = _plates(n)
+    first = _solved(gpu, sc, a, b, fields, 1)
+    want = _solved(gpu, sc, a, b, fields, 4, 2)
+    once = _solved(gpu, sc, a, b, fields, 4)
+    assert np.max(np.abs(first["rot_w"] - once["rot_w"])) > 1e-4  # the later iterations matter
+    monkeypatch.setenv("DYPHUR_REFUSE_LAUNCH", str(refuse))
+    assert _same_bits(_solved(gpu, sc, a, b, fields, 4), once)
+    assert _same_bits(_solved(gpu, sc, a, b, fields, 4, 2), want)
