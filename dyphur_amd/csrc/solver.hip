@@ -1458,8 +1458,9 @@ __device__ __forceinline__ void st_words2(uint64_t *p, float a, float b, uint32_
 // (182 us) measured better than 32 (220) and 8 with twice the workgroups as 16.
 // Reading every word of a body that is one contact away (instead of two words
 // until they match) was slower from 32 768 bodies on (216 us).
+constexpr int kFirstThreads = 512;
 template <bool ONE_XCD>
-__global__ __launch_bounds__(512) void sweep_first(CRec rec, const uint4 *__restrict__ rseq, float *__restrict__ lam,
+__global__ __launch_bounds__(kFirstThreads) void sweep_first(CRec rec, const uint4 *__restrict__ rseq, float *__restrict__ lam,
                                                    uint64_t *bw, const float4 *__restrict__ sta, float mu, float dt,
                                                    uint32_t *meta) {
     uint32_t *err = meta + kMErr;
@@ -1791,6 +1792,7 @@ struct dy_xpbd_s {
         coop_lanes_max[2] = {0, 0}, coop_pair_max = 0, coop_first_max = 0, coop_motor_max = 0, device_cus = 0;
     int sweep_pair = 1;     // contact-only dataflow sweeps use sweep_flow_pair (DYPHUR_SWEEP_PAIR=0: sweep_flow)
     int pair_threads = 512;  // its workgroup size (DYPHUR_SWEEP_PAIR_THREADS)
+    int first_threads = 512;  // sweep_first's: the same, at most its launch bound
     // Constraint capacity (contacts + joints) of the constraint-indexed
     // buffers, and the joint capacity of jpk / jend.
     uint32_t ccap = 0, jcap = 0;
@@ -1966,6 +1968,7 @@ int query_coop(dy_xpbd_s *x) {
     {
         const int pt = env_int("DYPHUR_SWEEP_PAIR_THREADS", 512);
         x->pair_threads = (pt == 128 || pt == 256 || pt == 512 || pt == 1024) ? pt : 512;
+        x->first_threads = x->pair_threads < kFirstThreads ? x->pair_threads : kFirstThreads;
     }
     if (!coop) return DY_OK;
     int per_cu = 0;
@@ -1994,9 +1997,9 @@ int query_coop(dy_xpbd_s *x) {
                                                         x->pair_threads, 0));
     x->coop_pair_max = per_cu * x->device_cus;
     DY_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(sweep_first<false>),
-                                                        x->pair_threads, 0));
+                                                        x->first_threads, 0));
     DY_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_xcd, reinterpret_cast<const void *>(sweep_first<true>),
-                                                        x->pair_threads, 0));
+                                                        x->first_threads, 0));
     x->coop_first_max = (per_cu < per_cu_xcd ? per_cu : per_cu_xcd) * x->device_cus;
     return DY_OK;
 }
@@ -2249,7 +2252,7 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
         // a workgroup per CU, of the chip or of the one XCD (an eighth of the launch)
         const bool one_xcd = nb <= kSweepOneXcd;
         const int dflt = one_xcd ? x->device_cus / 8 : x->device_cus;
-        uint32_t blocks = coop_blocks(x, x->sweep_blocks_override > 0 ? x->sweep_blocks_override : dflt, x->pair_threads,
+        uint32_t blocks = coop_blocks(x, x->sweep_blocks_override > 0 ? x->sweep_blocks_override : dflt, x->first_threads,
                                       x->coop_first_max);
         if (one_xcd) blocks *= 8u;
         if (blocks > static_cast<uint32_t>(x->coop_first_max)) blocks = static_cast<uint32_t>(x->coop_first_max);
@@ -2263,7 +2266,7 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
         if (!grid_launch(x, 4,
                          one_xcd ? reinterpret_cast<const void *>(sweep_first<true>)
                                  : reinterpret_cast<const void *>(sweep_first<false>),
-                         blocks, x->pair_threads, args, st)) {
+                         blocks, x->first_threads, args, st)) {
             x->coop_refused = true;
             coop = false;
             words = false;

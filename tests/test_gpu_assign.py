@@ -180,3 +180,31 @@ def test_refused_launches_change_nothing(gpu, monkeypatch, n, refuse):
     monkeypatch.setenv("DYPHUR_REFUSE_LAUNCH", str(refuse))
     assert _same_bits(_solved(gpu, sc, a, b, fields, 4), once)
     assert _same_bits(_solved(gpu, sc, a, b, fields, 4, 2), want)
+
+
+@pytest.mark.parametrize("threads", [128, 256, 1024])
+def test_pair_threads_launch_as_asked(gpu, monkeypatch, threads):
+    """Every accepted DYPHUR_SWEEP_PAIR_THREADS launches: a refused one would
+    leave the solver to launches per round and per class with the host between
+    them, which take more than ten times as long."""
+    n, nc = 5000, 15000
+    a, b, _, sc = _contacts(n, nc)
+    rng = np.random.default_rng(1)
+    normal = rng.normal(size=(3, nc))
+    normal /= np.linalg.norm(normal, axis=0)
+    fields = [v.astype(np.float32) for v in (*sc.pos[a].T, *normal, rng.uniform(0.0, 0.01, nc))]
+    ms = []
+    for t in (512, threads):
+        monkeypatch.setenv("DYPHUR_SWEEP_PAIR_THREADS", str(t))
+        print(f"[pair threads] {t}", flush=True)
+        s = gpu.Stream()
+        db = gpu.DeviceBodies(sc, s)
+        solver = gpu.XpbdSolver(s, 10, nc, 0.5)
+        cv, _keep = _view(gpu, s, a, b, fields)
+        solver.solve(s, cv, db, sc.dt)
+        solver.set_timing(True)
+        for _ in range(10):
+            solver.solve(s, cv, db, sc.dt)
+        tm = solver.timing(s)
+        ms.append((tm["assign_ms"] + tm["sweep_ms"]) / tm["solves"])
+    assert ms[1] < 4.0 * ms[0], ms

@@ -295,6 +295,9 @@ LAUNCH_SHAPES = [
     ("sweep_phases_one_xcd", {"DYPHUR_SWEEP_MODE": "0"}),
     ("sweep_phases_one_block", {"DYPHUR_SWEEP_MODE": "0", "DYPHUR_SWEEP_BLOCKS": "1"}),
     ("sweep_dataflow_lane_cursors", {"DYPHUR_SWEEP_MODE": "3"}),
+    ("sweep_pair_wg128", {"DYPHUR_SWEEP_PAIR_THREADS": "128"}),
+    ("sweep_pair_wg256", {"DYPHUR_SWEEP_PAIR_THREADS": "256"}),
+    ("sweep_pair_wg1024", {"DYPHUR_SWEEP_PAIR_THREADS": "1024"}),
     ("sweep_dataflow_lane_cursors_one_block", {"DYPHUR_SWEEP_MODE": "3", "DYPHUR_SWEEP_BLOCKS": "1"}),
 ]
 
