@@ -83,6 +83,7 @@ enum : uint32_t {
     kMFcnt = 20,         // 3 words: frontier sizes
     kMRegSweep = 24,     // 2 words: check-in of sweep_xcd (participants, arrivals)
     kMFree = 26,         // constraints between two static bodies
+    kMSelf = 27,         // a contact names one dynamic body twice
     kMRegMotor = 28,     // 2 words: check-in of joint_motors_xcd
     kMBarMotor = 30,     // 2 words: barrier of joint_motors_xcd
     kMRegAssign = 32,    // 2 words: check-in of assign_flow on one XCD
@@ -283,7 +284,8 @@ __global__ void solve_degree(Cons cs, const uint32_t *__restrict__ meta, const f
 }
 
 // Unordered per-body lists of dynamic endpoints: adj = (c << 1 | end), own = body.
-// Constraints between two static bodies get class 0 and round 1 here.
+// Constraints between two static bodies get class 0 and round 1 here.  A
+// contact of a dynamic body with itself is noted: it would wait for itself.
 __global__ void solve_fill(Cons cs, uint32_t *__restrict__ meta, const float *__restrict__ im,
                            const uint32_t *__restrict__ off, uint32_t *__restrict__ fill, uint32_t *__restrict__ adj,
                            uint32_t *__restrict__ own, uint32_t *__restrict__ cstat, uint64_t *__restrict__ state) {
@@ -315,6 +317,8 @@ __global__ void solve_fill(Cons cs, uint32_t *__restrict__ meta, const float *__
             if (a == kNone && b == kNone) {
                 state[c] = 1ull << 32;
                 atomicAdd(&meta[kMFree], 1u);
+            } else if (a == b) {
+                meta[kMSelf] = 1u;
             }
         }
     }
@@ -780,7 +784,8 @@ __global__ __launch_bounds__(1024) void assign_flow(AssignBufs B) {
         if (threadIdx.x < 3u) s_stat[threadIdx.x] = 0u;
         __syncthreads();
         AssignStats S{0u, 0u, 0u};
-        (void)flow_bodies<ONE_XCD>(B, serial, gtid, stride, lhist, S);  // a timeout leaves contacts unassigned: kErrAssign
+        // a contact of a body with itself, and a timeout, leave contacts unassigned: kErrAssign
+        if (meta[kMSelf] == 0u) (void)flow_bodies<ONE_XCD>(B, serial, gtid, stride, lhist, S);
         if (gtid == 0) {
             // constraints between two static bodies are on no list: class 0, round 1 (solve_fill)
             const uint32_t free_ones = meta[kMFree];

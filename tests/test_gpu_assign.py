@@ -208,3 +208,29 @@ def test_pair_threads_launch_as_asked(gpu, monkeypatch, threads):
         tm = solver.timing(s)
         ms.append((tm["assign_ms"] + tm["sweep_ms"]) / tm["solves"])
     assert ms[1] < 4.0 * ms[0], ms
+
+
+@pytest.mark.parametrize("n,nc,serial", [(50, 100, False), (1000, 3000, False), (1000, 3000, True), (16400, 30000, False)])
+def test_contact_of_a_body_with_itself_is_an_error_at_once(gpu, n, nc, serial):
+    """No list order lets such a contact go first; the solve reports it without
+    waiting for the kernels' limits, and leaves the bodies where they were."""
+    import time
+    print(f"[self contact] n={n} nc={nc} serial={serial}", flush=True)
+    a, b, static, sc = _contacts(n, nc)
+    k = int(np.nonzero(~static[a])[0][nc // 3])
+    b[k] = a[k]
+    z = np.zeros(nc, np.float32)
+    s = gpu.Stream()
+    db = gpu.DeviceBodies(sc, s)
+    solver = gpu.XpbdSolver(s, 3, nc, 0.5)
+    solver.set_force_serial(serial)
+    cv, _keep = _view(gpu, s, a, b, [z] * 6 + [z + np.float32(0.01)])
+    before = db.download(s)
+    t0 = time.perf_counter()
+    solver.solve(s, cv, db, sc.dt)
+    with pytest.raises(gpu.DyError):
+        solver.stats()
+    assert time.perf_counter() - t0 < 0.5
+    after = db.download(s)
+    for f in ("pos_x", "pos_y", "pos_z", "vel_x", "vel_y", "vel_z"):
+        assert np.array_equal(before[f], after[f]), f
