@@ -1793,7 +1793,7 @@ struct dy_xpbd_s {
     dy_solve_stats stats{};
     // Co-resident workgroup limits of the cooperative kernels, [0] contacts
     // only, [1] the variants that also solve joints.
-    int coop_assign_max = 0, coop_sweep_max[2] = {0, 0}, coop_xcd_max[2] = {0, 0}, coop_flow_max[2] = {0, 0},
+    int coop_assign_max = 0, assign_most = 0, coop_sweep_max[2] = {0, 0}, coop_xcd_max[2] = {0, 0}, coop_flow_max[2] = {0, 0},
         coop_lanes_max[2] = {0, 0}, coop_pair_max = 0, coop_first_max = 0, coop_motor_max = 0, device_cus = 0;
     int sweep_pair = 1;     // contact-only dataflow sweeps use sweep_flow_pair (DYPHUR_SWEEP_PAIR=0: sweep_flow)
     int pair_threads = 512;  // its workgroup size (DYPHUR_SWEEP_PAIR_THREADS)
@@ -1982,7 +1982,9 @@ int query_coop(dy_xpbd_s *x) {
                                                         x->assign_threads, 0));
     DY_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_xcd, reinterpret_cast<const void *>(assign_flow<true>),
                                                         x->assign_threads, 0));
-    x->coop_assign_max = (per_cu < per_cu_xcd ? per_cu : per_cu_xcd) * x->device_cus;
+    per_cu = per_cu < per_cu_xcd ? per_cu : per_cu_xcd;
+    x->coop_assign_max = per_cu * x->device_cus;
+    x->assign_most = per_cu > 2 ? (per_cu - 1) / 2 * x->device_cus : (x->coop_assign_max > 1 ? x->coop_assign_max / 2 : 1);
     const void *fns[4][2] = {
         {reinterpret_cast<const void *>(sweep_persistent<false>), reinterpret_cast<const void *>(sweep_persistent<true>)},
         {reinterpret_cast<const void *>(sweep_xcd<false>), reinterpret_cast<const void *>(sweep_xcd<true>)},
@@ -2190,11 +2192,15 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
         AssignBufs B{x->adj, x->own, x->off.p, x->deg.p, x->cstat, x->slot, x->flow, x->used.p, x->state, x->meta,
                      x->hist, x->boff, x->bfill, nb};
         void *args[] = {&B};
-        // A thread per body, as far as half of what the occupancy query promises
-        // holds them: the workgroups wait for each other, and the query has
-        // named one or two workgroups a CU more than were resident.
+        // A thread per body, as far as half of what is resident holds them: the
+        // workgroups wait for each other, and so do another solver's on another
+        // stream.  The occupancy query has named one workgroup a CU more than was
+        // resident.  3 workgroups of 256 a CU (12 of 24 wavefronts) leave a CU room
+        // for sweep_first's (8) wherever they land, and for the same again.  Bodies
+        // past those threads go several a thread: 200 000 bodies 184 us with room
+        // for them all, 233 so, 300 000 238 against 220.
         const bool one_xcd = nb <= kAssignOneXcd;
-        const uint32_t most = static_cast<uint32_t>(x->coop_assign_max > 1 ? x->coop_assign_max / 2 : 1);
+        const uint32_t most = static_cast<uint32_t>(x->assign_most);
         uint32_t blocks = x->assign_blocks_override > 0 ? static_cast<uint32_t>(x->assign_blocks_override)
                                                         : ceil_div(nb ? nb : 1u, static_cast<uint32_t>(x->assign_threads));
         if (one_xcd) blocks *= 8u;  // an eighth of a launch runs on the XCD

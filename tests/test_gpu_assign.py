@@ -234,3 +234,26 @@ def test_contact_of_a_body_with_itself_is_an_error_at_once(gpu, n, nc, serial):
     after = db.download(s)
     for f in ("pos_x", "pos_y", "pos_z", "vel_x", "vel_y", "vel_z"):
         assert np.array_equal(before[f], after[f]), f
+
+
+def test_two_large_worlds_on_two_streams(gpu):
+    """Two worlds past 16 384 bodies step side by side, each on its own stream:
+    the kernels whose workgroups wait for each other leave room for another
+    world's, and both worlds go as they go alone."""
+    scs = [scenes.random_mixed(20000, seed=k, extent=(26, 20, 26)) for k in (3, 4)]
+    frames = 12
+    alone = []
+    for sc in scs:
+        w = gpu.World(sc)
+        for _ in range(frames):
+            w.step_async()
+        w.check()
+        alone.append(w.fnv())
+    print("[two worlds] side by side", flush=True)
+    worlds = [gpu.World(sc) for sc in scs]
+    for _ in range(frames):
+        for w in worlds:
+            w.step_async()
+    for w in worlds:
+        w.check()
+    assert [w.fnv() for w in worlds] == alone
