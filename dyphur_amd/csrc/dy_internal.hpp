@@ -197,12 +197,9 @@ __device__ __forceinline__ T ld_agent(const T *p) {
 }
 
 // Barrier among the nblk workgroups of one XCD (bar[0] arrivals, bar[1]
-// generation; zero before the launch).  With `fence`, thread 0 also acquires
-// at agent scope after the wait, so that plain loads after the barrier see
-// data written before it by the other workgroups.  False on a timeout (err
-// gets err_bit).
+// generation; zero before the launch).  False on a timeout (err gets err_bit).
 __device__ __forceinline__ bool xcd_barrier(uint32_t *bar, uint32_t &gen, uint32_t nblk, uint32_t *err,
-                                            uint32_t err_bit, bool fence = false) {
+                                            uint32_t err_bit) {
     __shared__ uint32_t s_ok;
     wait_vmem();
     __syncthreads();
@@ -226,7 +223,6 @@ __device__ __forceinline__ bool xcd_barrier(uint32_t *bar, uint32_t &gen, uint32
                 }
             }
         }
-        if (fence) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         s_ok = ok;
     }
     gen += 1u;

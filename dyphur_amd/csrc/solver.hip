@@ -1558,15 +1558,15 @@ __global__ __launch_bounds__(kFirstThreads) void sweep_first(CRec rec, const uin
 // 2k + 1 of a wave take record i0 + k, one body each, project_contact_pair):
 // each lane polls, loads, renormalises, stores and publishes its own body,
 // so a pass of the projection is about half as long.  Otherwise sweep_flow.
-// With `bw`, sweep_first has done iteration 0: nothing is left to do unless a
-// contact is still live, and then the bodies' records are made from their words.
+// sweep_first has done iteration 0: nothing is left to do unless a contact is
+// still live, and then the bodies' records are made from their words first.
 __global__ __launch_bounds__(1024) void sweep_flow_pair(uint32_t n_iters, CRec rec, const uint4 *__restrict__ rseq,
                                                         float *__restrict__ lam, float4 *__restrict__ dyn,
                                                         const float4 *__restrict__ sta, uint32_t *ver, float mu,
                                                         float dt, uint32_t *meta,
                                                         const uint64_t *__restrict__ bw, uint32_t nb) {
     uint32_t *err = meta + kMErr;
-    if (bw && meta[kMLive] == 0u) return;
+    if (meta[kMLive] == 0u) return;
     uint32_t bidx = 0, nblk = 0;
     if (!xcd_checkin(kSweepXcc, meta + kMRegSweep, err, kErrBarrier, bidx, nblk)) return;
     if (meta[kMErr] & kErrAssign) return;
@@ -1575,19 +1575,13 @@ __global__ __launch_bounds__(1024) void sweep_flow_pair(uint32_t n_iters, CRec r
     const uint32_t lane = lane_id(), side = lane & 1u;
     const uint32_t wave_rec0 = (bidx * blockDim.x + (threadIdx.x & ~63u)) / 2u;
     uint32_t gen = 0;
-    if (bw) {
-        for (uint32_t i = bidx * blockDim.x + threadIdx.x; i < nb; i += nblk * blockDim.x) {
-            uint32_t tag;
-            store_aos(dyn, i, words_state(bw, i, tag), 0u);
-            ver[i] = tag;
-        }
-        if (!xcd_barrier(meta + kMBarSweep, gen, nblk, err, kErrBarrier)) return;
+    for (uint32_t i = bidx * blockDim.x + threadIdx.x; i < nb; i += nblk * blockDim.x) {
+        uint32_t tag;
+        store_aos(dyn, i, words_state(bw, i, tag), 0u);
+        ver[i] = tag;
     }
-    for (uint32_t it = bw ? 1u : 0u; it < n_iters; ++it) {
-        if (it == 1 && !bw) {
-            if (!xcd_barrier(meta + kMBarSweep, gen, nblk, err, kErrBarrier)) return;
-            if (ld_agent(&meta[kMLive]) == 0u) return;
-        }
+    if (!xcd_barrier(meta + kMBarSweep, gen, nblk, err, kErrBarrier)) return;
+    for (uint32_t it = 1; it < n_iters; ++it) {
         for (uint32_t r0 = wave_rec0; r0 < nc; r0 += rstride) {
             const uint32_t i = r0 + (lane >> 1);
             bool todo = i < nc;  // the same on both lanes of a pair
@@ -1621,7 +1615,6 @@ __global__ __launch_bounds__(1024) void sweep_flow_pair(uint32_t n_iters, CRec r
                     project_contact_pair(ci, S, side, mu, l, dt, [](float v) { return __shfl_xor(v, 1, 64); });
                     if (side == 0u) lam[i] = l;
                     if (S.im != 0.f) store_aos(dyn, x, S, it);
-                    if (side == 0u && it == 0 && contact_live(p1.z, l)) atomicOr(&meta[kMLive], 1u);
                 }
                 if (ready) todo = false;
                 wait_vmem();  // body stores acknowledged by the L2 before the versions move
@@ -2307,7 +2300,7 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
         const float4 *stav = x->sta.p;
         uint32_t *verv = x->ver.p, *metav = x->meta;
         float muv = x->mu, dtv = dt;
-        const uint64_t *bwv = words ? x->bw.p : nullptr;
+        const uint64_t *bwv = x->bw.p;
         uint32_t nbv = nb;
         void *args_pair[] = {&iv, &rec, &rseqv, &lamv, &dynv, &stav, &verv, &muv, &dtv, &metav, &bwv, &nbv};
         void *args_flow[] = {&iv, &rec, &rseqv, &lamv, &dynv, &stav, &verv, &muv, &dtv, &metav, &jpkv};
