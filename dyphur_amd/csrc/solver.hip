@@ -1764,8 +1764,9 @@ struct dy_xpbd_s {
     uint32_t cap = 0;
     float *lam = nullptr;
     uint64_t *state = nullptr;
-    uint32_t *adj = nullptr, *own = nullptr, *crank = nullptr, *cstat = nullptr, *pending = nullptr;
-    uint32_t *fr0 = nullptr, *fr1 = nullptr;
+    uint32_t *adj = nullptr, *own = nullptr, *cstat = nullptr;
+    // launches per round only, made by the first solve that takes them
+    uint32_t *crank = nullptr, *pending = nullptr, *fr0 = nullptr, *fr1 = nullptr;
     uint32_t *boff = nullptr, *bfill = nullptr, *hist = nullptr, *rec_id = nullptr, *cpos = nullptr;
     uint32_t *meta = nullptr;  // kMWords device words
     uint4 *lrec = nullptr, *rseq = nullptr;
@@ -1830,7 +1831,6 @@ int sync_meta(dy_xpbd_s *x) {
     x->stats.rounds = m[kMRounds];
     x->stats.overflow = m[kMOverflow];
     x->stats.dyn_endpoints = m[kMDyn];
-
     if (m[kMErr] == kErrJoint) return DY_ERR_INVALID_ARG;
     return m[kMErr] ? DY_ERR_INTERNAL : DY_OK;
 }
@@ -1855,7 +1855,9 @@ int collect_timing(dy_xpbd_s *x) {
     return DY_OK;
 }
 
-// The constraint-indexed buffers, for c constraints (contacts + joints).
+// The constraint-indexed buffers, for c constraints (contacts + joints): 156
+// bytes each, with the 32 of the flow words and the 16 of the ordered lists;
+// per body there are 128 of words, 96 of records and 32 of counters and masks.
 void free_constraint_bufs(dy_xpbd_s *x) {
     void **ptrs[] = {(void **)&x->lam, (void **)&x->state, (void **)&x->adj, (void **)&x->own, (void **)&x->slot,
                      (void **)&x->crank, (void **)&x->cstat, (void **)&x->pending, (void **)&x->fr0, (void **)&x->fr1,
@@ -1883,12 +1885,7 @@ hipError_t alloc_constraint_bufs(dy_xpbd_s *x, uint32_t n_con) {
     dalloc(x->adj, 2 * c);
     dalloc(x->own, 2 * c);
     dalloc(x->slot, 2 * c);
-    dalloc(x->crank, 2 * c);
     dalloc(x->cstat, c);
-    dalloc(x->pending, c);
-    dalloc(x->fr0, c);
-    dalloc(x->fr1, c);
-    dalloc(x->lrec, c);
     dalloc(x->flow, 2 * c);
     dalloc(x->boff, ncls);
     dalloc(x->bfill, ncls);
@@ -1901,6 +1898,22 @@ hipError_t alloc_constraint_bufs(dy_xpbd_s *x, uint32_t n_con) {
     dalloc(x->rec_p1, c);
     if (e == hipSuccess) x->ccap = static_cast<uint32_t>(c);
     return e;
+}
+
+// The buffers of the launch-per-round assignment (36 bytes a constraint), which
+// synchronises with the host in any case.
+int ensure_rounds(dy_xpbd_s *x) {
+    const size_t c = x->ccap;
+    hipError_t e = hipSuccess;
+    auto dalloc = [&e](auto *&p, size_t n) {
+        if (!p && e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&p), n * sizeof(*p));
+    };
+    dalloc(x->crank, 2 * c);
+    dalloc(x->pending, c);
+    dalloc(x->fr0, c);
+    dalloc(x->fr1, c);
+    dalloc(x->lrec, c);
+    return static_cast<int>(e);
 }
 
 // Room for nj joints: joint parameters and the constraint buffers for
@@ -2023,6 +2036,7 @@ bool grid_launch(const dy_xpbd_s *x, int kind, const void *fn, uint32_t blocks, 
 // Launch-per-round assignment: the host drives the rounds and decides the
 // fallback to the reference order, reading the metadata every 16 rounds.
 int assign_by_rounds(dy_xpbd_s *x, hipStream_t st, const Cons &cv, const float *im) {
+    DY_TRY_STATUS(ensure_rounds(x));
     uint32_t h[kMWords];
     for (int pass = 0; pass < 2; ++pass) {
         const uint32_t cap = x->cap + x->jcap;

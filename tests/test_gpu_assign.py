@@ -257,3 +257,24 @@ def test_two_large_worlds_on_two_streams(gpu):
     for w in worlds:
         w.check()
     assert [w.fnv() for w in worlds] == alone
+
+
+def test_solver_memory_per_contact(gpu):
+    """A solver takes 156 bytes a contact; the launches per round take 36 more
+    only when a solve needs them."""
+    import ctypes
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+
+    def left():
+        assert gpu.lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    s = gpu.Stream()
+    gpu.XpbdSolver(s, 2, 1000, 0.5).close()
+    n = 16 << 20
+    before = left()
+    solver = gpu.XpbdSolver(s, 2, n, 0.5)
+    took = before - left()
+    solver.close()
+    print(f"[solver memory] {took / n:.1f} bytes a contact", flush=True)
+    assert 150 * n < took < 162 * n
