@@ -40,6 +40,7 @@
 #include <utility>
 #include <vector>
 
+#include "batch_shape.hpp"
 #include "dy_internal.hpp"
 #include "pair_contact.hpp"
 #include "adjoint.hpp"
@@ -1510,6 +1511,7 @@ struct dy_batch_s {
         Units glob;  // the others: state in global memory
     };
     uint32_t n_scenes = 0, max_n = 0, block = 256, wave_max = 128;
+    uint32_t wave_max_rec = 128;  // wave_max of recording launches (fewer workgroups fit at once)
     uint32_t lds_max_floats = kLdsMaxFloats;  // dynamic LDS one workgroup may take on this device
     int n_iters = 10;
     float mu = 0.5f;
@@ -1674,14 +1676,14 @@ BatchArgs batch_args(dy_batch_s *b, const dy_body_view &bodies, const dy_shape_v
 // read once and written back at the end): a recompute can then read a
 // checkpoint in place.
 bool batch_tape_ok(const dy_batch_s *b) {
-    const auto it = b->shapes.find(std::make_pair(b->block, b->wave_max));
+    const auto it = b->shapes.find(std::make_pair(b->block, b->wave_max_rec));
     return it != b->shapes.end() && it->second.glob.n_units == 0;
 }
 
 int batch_launch(dy_batch_s *b, hipStream_t s, const dy_body_view &bodies, const dy_shape_view &shapes, float gx,
                  float gy, float gz, float dt, int n_substeps, int n_frames, float *tape = nullptr,
                  const uint64_t *tape_off = nullptr, bool keep_input = false, const uint32_t *tape_cap = nullptr) {
-    const auto it = b->shapes.find(std::make_pair(b->block, b->wave_max));
+    const auto it = b->shapes.find(std::make_pair(b->block, tape ? b->wave_max_rec : b->wave_max));
     if (it == b->shapes.end()) return DY_ERR_INTERNAL;
     const dy_batch_s::Shape &sh = it->second;
     BatchArgs a = batch_args(b, bodies, shapes, gx, gy, gz, dt, n_substeps, n_frames);
@@ -1833,20 +1835,21 @@ int dy_batch_create(dy_stream_t s, uint32_t n_scenes, const uint32_t *body_offse
         if (hipEventCreateWithFlags(e, hipEventDisableTiming) != hipSuccess) return fail(DY_ERR_INTERNAL);
     {
         // dynamic LDS one workgroup may take, less 4 KiB for the kernels' static LDS
-        int dev = 0, lds = 0, cus = 0;
+        int dev = 0, lds = 0, cus = 0, per_cu = 0, per_cu_rec = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, reinterpret_cast<const void *>(batch_frames<256, false, true, false>), 256, 0) != hipSuccess ||
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu_rec, reinterpret_cast<const void *>(batch_frames<256, false, true, true>), 256, 0) != hipSuccess)
             return fail(DY_ERR_INTERNAL);
-        // Few scenes leave CUs idle and the longest scene decides: scenes past 32
-        // bodies get a workgroup each.  Many fill the chip: a wavefront each up to
-        // 128 bodies.  10 frames of 16 scenes of up to 256 bodies 1 670 -> 1 110 us,
-        // 300 scenes 2 340 -> 2 220, 600 2 490 -> 2 310, 1 200 2 690 -> 2 580, but
-        // 2 400 3 240 -> 4 370: the line is at 4 scenes a CU.
-        if (n_scenes <= 4u * static_cast<uint32_t>(cus)) b->wave_max = 32;
+        b->wave_max = batch_wave_max(b->body_off.data(), n_scenes, static_cast<uint32_t>(per_cu * cus));
+        b->wave_max_rec = batch_wave_max(b->body_off.data(), n_scenes, static_cast<uint32_t>(per_cu_rec * cus));
         b->lds_max_floats = std::max<uint32_t>(kLdsMaxFloats, static_cast<uint32_t>(std::max(lds - 4096, 0)) / 4u);
     }
     DY_BATCH_TRY(prepare_shape(b, b->block, b->wave_max));
+    DY_BATCH_TRY(prepare_shape(b, b->block, b->wave_max_rec));
 #undef DY_BATCH_TRY
     *out = b;
     return DY_OK;
@@ -1870,7 +1873,7 @@ int dy_batch_set_shape(dy_batch_t b, uint32_t threads, uint32_t wave_scene_max) 
     if (threads == 64) wave_scene_max = 0;
     DY_TRY_STATUS(prepare_shape(b, threads, wave_scene_max));
     b->block = threads;
-    b->wave_max = wave_scene_max;
+    b->wave_max = b->wave_max_rec = wave_scene_max;
     return DY_OK;
 }
 
@@ -1891,7 +1894,8 @@ int dy_batch_set_lds_limit(dy_batch_t b, uint32_t bytes) {
         }
     b->shapes.clear();
     b->lds_max_floats = want;
-    return prepare_shape(b, b->block, b->wave_max);
+    DY_TRY_STATUS(prepare_shape(b, b->block, b->wave_max));
+    return prepare_shape(b, b->block, b->wave_max_rec);
 }
 
 int dy_batch_get_shape(dy_batch_t b, uint32_t *threads, uint32_t *wave_scene_max) {

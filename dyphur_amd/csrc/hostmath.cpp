@@ -2,6 +2,7 @@
 // host (hipcc --cuda-host-only), exported with a C ABI so the CPU test suite
 // can compare the exact code the kernels run against the oracle without a GPU.
 #include "adjoint.hpp"
+#include "batch_shape.hpp"
 #include "joint_math.hpp"
 
 #include <condition_variable>
@@ -523,4 +524,9 @@ extern "C" int hm_pair_projection_mismatches(int n, uint32_t seed) {
         bad += ok ? 0 : 1;
     }
     return bad;
+}
+
+// The batch's default wave_scene_max (batch_shape.hpp).
+extern "C" uint32_t hm_batch_wave_max(const uint32_t *off, uint32_t n_scenes, uint32_t slots) {
+    return batch_wave_max(off, n_scenes, slots);
 }

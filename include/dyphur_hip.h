@@ -406,8 +406,11 @@ int dy_batch_set_force_serial(dy_batch_t b, int force_serial);
 /* Launch shape of the step kernel: workgroup threads (64, 128 or 256) and the
  * largest scene (bodies, ground included) stepped by one wavefront; larger
  * scenes get a whole workgroup, smaller ones are packed threads/64 to a
- * workgroup.  Default 256 / 128, 256 / 32 for at most 4 scenes per CU.
- * Results do not depend on the shape. */
+ * workgroup.  Default 256 / 128, or 256 / 32 where the scenes past 32 bodies are
+ * few enough for the device to hold their workgroups (about 2 a CU when
+ * stepping, 1 when recording for a dy_diff_t, whose default is its own) and the
+ * longest of them decides.  Setting a shape sets it for both; get returns the
+ * stepping one.  Results do not depend on the shape. */
 int dy_batch_set_shape(dy_batch_t b, uint32_t threads, uint32_t wave_scene_max);
 int dy_batch_get_shape(dy_batch_t b, uint32_t *threads, uint32_t *wave_scene_max);
 /* LDS one workgroup of the step may take, in bytes (0: the device's maximum,

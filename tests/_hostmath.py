@@ -44,6 +44,8 @@ def lib():
         L.hm_atan2_cr.argtypes = [C.c_float, C.c_float]
         L.hm_atan2_cr_array.argtypes = [vp, vp, vp, C.c_size_t]
         L.hm_joint_pair.argtypes = [vp, vp, vp, C.c_uint32, C.c_float, C.c_int]
+        L.hm_batch_wave_max.restype = C.c_uint32
+        L.hm_batch_wave_max.argtypes = [vp, C.c_uint32, C.c_uint32]
         _lib = L
     return _lib
 
