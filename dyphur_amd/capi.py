@@ -861,11 +861,13 @@ class Batch(_Owned):
                                   sc.dt if dt is None else dt, sc.n_substeps if n_substeps is None else n_substeps,
                                   n_frames), "dy_batch_step")
 
-    TUNE_SHAPES = ((64, 0), (128, 64), (128, 128), (256, 64), (256, 128), (256, 256))
+    # the shapes that autotune times, and the default for few scenes, which it keeps where that is faster
+    TUNE_SHAPES = ((64, 0), (128, 64), (128, 128), (256, 64), (256, 128), (256, 256), (256, 32))
 
     def autotune(self, trial_frames: int = 5) -> tuple[tuple[int, int], list[float]]:
-        """Times the six launch shapes from the current state (which it
-        restores) and keeps the fastest; returns it and the six times in ms."""
+        """Times the six launch shapes, and the current one where it is none of
+        them, from the current state (which it restores) and keeps the fastest;
+        returns it and the six times in ms."""
         sc = self.scenes[0]
         g = sc.gravity
         bv, sv = self.bodies.view(), self.shapes.view()

@@ -1943,13 +1943,18 @@ int dy_batch_autotune(dy_batch_t b, dy_stream_t s, const dy_body_view *bodies, c
                               hipMemcpyDeviceToDevice, hsm));
         return DY_OK;
     };
-    const uint32_t cand[kTuneShapes][2] = {{64, 0}, {128, 64}, {128, 128}, {256, 64}, {256, 128}, {256, 256}};
+    // The six shapes, then the one the batch has where it is none of them.
+    const uint32_t keep[2] = {b->block, b->wave_max}, keep_rec = b->wave_max_rec;
+    const uint32_t cand[kTuneShapes + 1][2] = {{64, 0},   {128, 64},  {128, 128},        {256, 64},
+                                               {256, 128}, {256, 256}, {keep[0], keep[1]}};
+    uint32_t n_cand = kTuneShapes + 1;
+    for (uint32_t c = 0; c < kTuneShapes; ++c)
+        if (cand[c][0] == keep[0] && cand[c][1] == keep[1]) n_cand = kTuneShapes;
     float best = 0.f;
-    const uint32_t keep[2] = {b->block, b->wave_max};
-    uint32_t best_shape[2] = {keep[0], keep[1]};
+    uint32_t best_at = kTuneShapes;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) st = DY_ERR_INTERNAL;
     if (st == DY_OK) st = copy_state(true);
-    for (uint32_t c = 0; c < kTuneShapes && st == DY_OK; ++c) {
+    for (uint32_t c = 0; c < n_cand && st == DY_OK; ++c) {
         st = dy_batch_set_shape(b, cand[c][0], cand[c][1]);
         if (st == DY_OK) st = copy_state(false);
         if (st == DY_OK) st = batch_launch(b, hsm, *bodies, *shapes, gx, gy, gz, dt, n_substeps, 1);  // warm-up
@@ -1960,15 +1965,18 @@ int dy_batch_autotune(dy_batch_t b, dy_stream_t s, const dy_body_view *bodies, c
         if (st == DY_OK && hipEventSynchronize(e1) != hipSuccess) st = DY_ERR_INTERNAL;
         float ms = 0.f;
         if (st == DY_OK && hipEventElapsedTime(&ms, e0, e1) != hipSuccess) st = DY_ERR_INTERNAL;
-        if (ms_out) ms_out[c] = ms;
+        if (ms_out && c < kTuneShapes) ms_out[c] = ms;
         if (st == DY_OK && (c == 0 || ms < best)) {
             best = ms;
-            best_shape[0] = cand[c][0];
-            best_shape[1] = cand[c][1];
+            best_at = c;
         }
     }
-    if (st == DY_OK) st = dy_batch_set_shape(b, best_shape[0], best_shape[1]);
-    else (void)dy_batch_set_shape(b, keep[0], keep[1]);
+    if (st == DY_OK && best_at < kTuneShapes) {
+        st = dy_batch_set_shape(b, cand[best_at][0], cand[best_at][1]);
+    } else {
+        (void)dy_batch_set_shape(b, keep[0], keep[1]);
+        b->wave_max_rec = keep_rec;
+    }
     if (st == DY_OK) st = copy_state(false);
     if (hipStreamSynchronize(hsm) != hipSuccess && st == DY_OK) st = DY_ERR_INTERNAL;
     if (e0) (void)hipEventDestroy(e0);

@@ -429,10 +429,10 @@ int dy_batch_set_lds_limit(dy_batch_t b, uint32_t bytes);
 int dy_batch_step(dy_batch_t b, dy_stream_t s, const dy_body_view *bodies, const dy_shape_view *shapes,
                   float gx, float gy, float gz, float dt, int n_substeps, int n_frames);
 /* Times trial_frames frames at each of six launch shapes (threads /
- * wave_scene_max: 64/-, 128/64, 128/128, 256/64, 256/128, 256/256) from the
- * current state, keeps the fastest, and restores the body state and
- * statistics.  Blocking.  chosen_* (may be NULL) receive the shape; ms_out
- * (may be NULL) the six times in ms. */
+ * wave_scene_max: 64/-, 128/64, 128/128, 256/64, 256/128, 256/256), and at the
+ * batch's own shape where it is none of them, from the current state, keeps the
+ * fastest, and restores the body state and statistics.  Blocking.  chosen_*
+ * (may be NULL) receive the shape; ms_out (may be NULL) the six times in ms. */
 int dy_batch_autotune(dy_batch_t b, dy_stream_t s, const dy_body_view *bodies, const dy_shape_view *shapes,
                       float gx, float gy, float gz, float dt, int n_substeps, int trial_frames,
                       uint32_t *chosen_threads, uint32_t *chosen_wave_max, float *ms_out);

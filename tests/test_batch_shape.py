@@ -59,3 +59,19 @@ def test_default_shape_steps_and_records_as_any_other(gpu, n_scenes, n_dyn):
             assert np.array_equal(recorded[k].view(np.uint32), stepped[k].view(np.uint32)), k
         for k in adj:
             assert np.array_equal(adj[k].view(np.uint32), out[0][2][k].view(np.uint32)), k
+
+
+@pytest.mark.gpu
+def test_autotune_keeps_a_faster_shape_it_started_from(gpu):
+    """A batch for which the default beats the six shapes keeps it, recording
+    shape included; one that starts from one of the six takes the fastest of them."""
+    scs = [scenes.pile_scene(62, scenes.Pcg32(k)) for k in range(64)]
+    b = gpu.Batch(scs)
+    assert b.shape() == (256, 32) and b.shape() not in gpu.Batch.TUNE_SHAPES[:6]
+    b.step(40)
+    chosen, ms = b.autotune(8)
+    print(f"[autotune] kept {chosen}; the six: {[round(m, 3) for m in ms]} ms", flush=True)
+    assert chosen == b.shape() == (256, 32) and len(ms) == 6 and min(ms) > 0
+    b.set_shape(128, 64)
+    chosen, ms = b.autotune(8)
+    assert chosen == gpu.Batch.TUNE_SHAPES[int(np.argmin(ms))]
