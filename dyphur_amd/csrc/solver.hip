@@ -56,9 +56,9 @@ constexpr uint32_t kMaxGridBlocks = 1024;  // grid-stride kernels over capacity-
 // Bodies up to which assign_flow runs on one XCD (one XCD against the chip, mid-run piles: 2 000 bodies 38 against
 // 58 us, 5 000 54 / 81, 8 000 65 / 90, 12 000 80 / 101, 20 000 89 / 89, 32 768 250 / 98).
 constexpr uint32_t kAssignOneXcd = 16384;
-// The same line for sweep_first (one XCD against the chip: 1 024 boxes 45 against 52 us, 5 000 bodies 90 / 108,
-// 32 768 189 / 169, 98 305 457 / 254).
-constexpr uint32_t kSweepOneXcd = 16384;
+// sweep_first's line (one XCD against the chip, mid-run piles: 3 000 bodies 80 against 93 us, 8 000 114 / 146,
+// 12 000 129 / 162, 16 000 149 / 173, 20 000 164 / 179, 24 000 172 / 177, 32 768 189 / 169, 98 305 457 / 254).
+constexpr uint32_t kSweepOneXcd = 24576;
 constexpr uint32_t kSweepXcc = 0;         // the XCD whose workgroups run the assignment and the sweep
 
 // Solver metadata (device words).  solve_prep zeroes all but kMErr, which

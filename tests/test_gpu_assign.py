@@ -94,6 +94,7 @@ def test_classes_match_greedy(gpu, monkeypatch, n, nc, blocks, serial):
 @pytest.mark.parametrize("heavy", [False, True])
 @pytest.mark.parametrize("n,nc,iters,blocks", [
     (40, 33, 10, 0), (300, 257, 1, 0), (300, 900, 10, 1), (16384, 40001, 3, 0), (16385, 40001, 3, 0), (16385, 40001, 2, 2),
+    (24576, 60001, 3, 0), (24577, 60001, 3, 0), (24577, 40001, 2, 2),
 ])
 def test_first_iteration_by_words_matches_records(gpu, monkeypatch, n, nc, iters, blocks, heavy):
     """The sweep that hands bodies on as tagged words against the sweep over
@@ -165,7 +166,7 @@ def _same_bits(x, y):
     return all(np.array_equal(np.asarray(x[k]).view(np.uint32), np.asarray(y[k]).view(np.uint32)) for k in x)
 
 
-@pytest.mark.parametrize("n", [60, 3000, 16400])
+@pytest.mark.parametrize("n", [60, 3000, 24600])
 @pytest.mark.parametrize("refuse", [1, 4, 8])
 def test_refused_launches_change_nothing(gpu, monkeypatch, n, refuse):
     """A refused launch of the assignment (1), the first iteration (4) or the
@@ -237,10 +238,10 @@ def test_contact_of_a_body_with_itself_is_an_error_at_once(gpu, n, nc, serial):
 
 
 def test_two_large_worlds_on_two_streams(gpu):
-    """Two worlds past 16 384 bodies step side by side, each on its own stream:
+    """Two worlds of 26 000 bodies step side by side, each on its own stream:
     the kernels whose workgroups wait for each other leave room for another
     world's, and both worlds go as they go alone."""
-    scs = [scenes.random_mixed(20000, seed=k, extent=(26, 20, 26)) for k in (3, 4)]
+    scs = [scenes.random_mixed(26000, seed=k, extent=(26, 26, 26)) for k in (3, 4)]
     frames = 12
     alone = []
     for sc in scs:
