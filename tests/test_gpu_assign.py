@@ -8,20 +8,22 @@ from dyphur_amd import scenes
 pytestmark = pytest.mark.gpu
 
 
+def _jp_order(n):
+    """Contacts 0 .. n - 1 by falling priority."""
+    k = np.arange(n, dtype=np.uint64)
+    h = k.astype(np.uint32)
+    h ^= h >> np.uint32(16)
+    h *= np.uint32(0x85EBCA6B)
+    h ^= h >> np.uint32(13)
+    h *= np.uint32(0xC2B2AE35)
+    h ^= h >> np.uint32(16)
+    return np.argsort((h.astype(np.uint64) << np.uint64(32)) | k)[::-1]
+
+
 def _greedy(a, b, static, serial):
     """Classes by definition: in priority order (JP) the lowest colour free on
     both bodies, in index order one more than the bodies' levels."""
-    k = np.arange(len(a), dtype=np.uint64)
-    if serial:
-        order = np.arange(len(a))
-    else:
-        h = k.astype(np.uint32)
-        h ^= h >> np.uint32(16)
-        h *= np.uint32(0x85EBCA6B)
-        h ^= h >> np.uint32(13)
-        h *= np.uint32(0xC2B2AE35)
-        h ^= h >> np.uint32(16)
-        order = np.argsort((h.astype(np.uint64) << np.uint64(32)) | k)[::-1]
+    order = np.arange(len(a)) if serial else _jp_order(len(a))
     used = [0] * len(static)
     out = np.zeros(len(a), np.uint32)
     for c in order:
@@ -91,6 +93,43 @@ def test_classes_match_greedy(gpu, monkeypatch, n, nc, blocks, serial):
     assert np.array_equal(solver.classes(s, nc), ref)
 
 
+@pytest.mark.parametrize("n,nc,blocks", [(1000, 3000, 0), (16385, 40001, 0), (16385, 20000, 3), (30000, 20000, 0)])
+@pytest.mark.parametrize("kind", ["overflow", "deep"])
+def test_fallback_to_reference_order(gpu, monkeypatch, n, nc, blocks, kind):
+    """A body in more than 64 contacts that can see each other's colours, and a
+    chain of 300 rounds: the assignment ranks its lists again in contact order
+    inside the launch, on one XCD and over the chip, with one body a thread and
+    several."""
+    if blocks:
+        monkeypatch.setenv("DYPHUR_ASSIGN_BLOCKS", str(blocks))
+    print(f"[assign fallback] {kind} n={n} nc={nc} blocks={blocks}", flush=True)
+    a, b, static, sc = _contacts(n, nc)
+    free = np.nonzero(~static)[0]
+    if kind == "overflow":
+        hub = free[len(free) // 2]
+        at = np.arange(0, nc, nc // 150)
+        a[at], b[at] = hub, free[: len(at)]
+        a[at[b[at] == hub]] = free[-1]
+    else:
+        at = _jp_order(nc)[:300]  # contact at[k] waits for at[k - 1]
+        chain = free[-301:]
+        used = np.isin(a, chain) | np.isin(b, chain)
+        a[used], b[used] = free[0], free[1]
+        a[at], b[at] = chain[:-1], chain[1:]
+    s = gpu.Stream()
+    db = gpu.DeviceBodies(sc, s)
+    solver = gpu.XpbdSolver(s, 2, nc, 0.5)
+    z = np.zeros(nc, np.float32)
+    cv, _keep = _view(gpu, s, a, b, [z] * 7)
+    ref = _greedy(a, b, static, True)
+    for _ in range(2):
+        solver.solve(s, cv, db, sc.dt)
+        st = solver.stats()
+        assert st["used_serial"] == 1 and st["overflow"] == (1 if kind == "overflow" else st["overflow"])
+        assert st["n_constraints"] == nc and st["n_classes"] == ref.max() + 1
+        assert np.array_equal(solver.classes(s, nc), ref)
+
+
 @pytest.mark.parametrize("heavy", [False, True])
 @pytest.mark.parametrize("n,nc,iters,blocks", [
     (40, 33, 10, 0), (300, 257, 1, 0), (300, 900, 10, 1), (16384, 40001, 3, 0), (16385, 40001, 3, 0), (16385, 40001, 2, 2),
@@ -99,7 +138,8 @@ def test_classes_match_greedy(gpu, monkeypatch, n, nc, blocks, serial):
 def test_first_iteration_by_words_matches_records(gpu, monkeypatch, n, nc, iters, blocks, heavy):
     """The sweep that hands bodies on as tagged words against the sweep over
     acknowledged records, bit for bit.  Contacts between bodies of almost no
-    inverse mass stay live after the first iteration, so the later ones run."""
+    inverse mass stay live after the first iteration, so the later ones run
+    (test_later_iterations_by_words has such contacts move)."""
     if blocks:
         monkeypatch.setenv("DYPHUR_SWEEP_BLOCKS", str(blocks))
     rng = np.random.default_rng(7)
@@ -279,3 +319,17 @@ def test_solver_memory_per_contact(gpu):
     solver.close()
     print(f"[solver memory] {took / n:.1f} bytes a contact", flush=True)
     assert 150 * n < took < 162 * n
+
+
+@pytest.mark.parametrize("n,iters", [(60, 2), (3000, 4), (24600, 3)])
+def test_later_iterations_by_words(gpu, monkeypatch, n, iters):
+    """Contacts that the first iteration leaves live and the later ones move:
+    the records made from the words, against the sweep over records."""
+    print(f"[later iterations] n={n} iters={iters}", flush=True)
+    sc, a, b, fields = _plates(n)
+    first = _solved(gpu, sc, a, b, fields, 1)
+    got = _solved(gpu, sc, a, b, fields, iters, 2)
+    once = _solved(gpu, sc, a, b, fields, iters)
+    assert np.max(np.abs(first["rot_w"] - once["rot_w"])) > 1e-4
+    monkeypatch.setenv("DYPHUR_SWEEP_PAIR", "0")
+    assert _same_bits(_solved(gpu, sc, a, b, fields, iters, 2), got)

@@ -252,11 +252,15 @@ def test_exclusive_scan_sizes(gpu, n):
     assert int(dtot.download(s)[0]) == int(a.sum(dtype=np.uint64))
 
 
-def test_cooperative_launch_path_identical(gpu, monkeypatch):
-    """The grid-synchronised kernels (Morton sort, class assignment, sweep)
-    give the same frames launched as ordinary launches (the default) and
-    through the runtime's cooperative path (DYPHUR_COOP_LAUNCH=1)."""
-    sc = scenes.random_mixed(12000, seed=11, extent=(24, 14, 24))
+@pytest.mark.parametrize("n,sort_blocks", [(12000, None), (26000, "64")])
+def test_cooperative_launch_path_identical(gpu, monkeypatch, n, sort_blocks):
+    """The grid-synchronised kernels (class assignment and sweeps, on one XCD
+    and over the chip, and the Morton sort where it is asked for) give the same
+    frames launched as ordinary launches (the default) and through the
+    runtime's cooperative path (DYPHUR_COOP_LAUNCH=1)."""
+    sc = scenes.random_mixed(n, seed=11, extent=(24, n / 857.0, 24))
+    if sort_blocks:
+        monkeypatch.setenv("DYPHUR_SORT_BLOCKS", sort_blocks)
     hs = []
     for coop in ("0", "1"):
         monkeypatch.setenv("DYPHUR_COOP_LAUNCH", coop)
