@@ -208,7 +208,10 @@ def stage_kernels(capi, w, sc, s, n_frames: int) -> dict:
     world's current state (untimed: the stage events and the solver's kernel
     timing wait on the host every frame).  Returns {kernel: (ms per launch,
     bytes per launch)}; the broadphase's launches come from its own kernel
-    timing, integrate and the narrowphase from events around their calls."""
+    timing, integrate and the narrowphase from events around their calls.  A
+    name stands for its stage: rank_sort is rank_tiles, rank_merge and
+    rank_scatter, assign_flow includes list_rank, sweep_first the check
+    whether a contact is left live."""
     n = sc.n
     n_static = int(np.count_nonzero(sc.flags & 1))
     e = [capi.Event() for _ in range(4)]
@@ -243,14 +246,14 @@ def stage_kernels(capi, w, sc, s, n_frames: int) -> dict:
     ns = float(max(tm["solves"], 1))
     return {
         "integrate_kernel": (integ / f, 100.0 * (n - n_static) + 4.0 * n_static),
-        "morton_sort_grid": (bt["sort_ms"] / nb, 48.0 * n),
+        "rank_sort": (bt["sort_ms"] / nb, 48.0 * n),
         "karras_build": (bt["karras_ms"] / nb, 24.0 * n),
         "leaf_refit": (bt["refit_ms"] / nb, 108.0 * n),
         "traverse_count": (bt["traverse_ms"] / nb, 52.0 * n),
         "emit_pairs": (bt["emit_ms"] / nb, 8.0 * P),
         "narrowphase": (narrow / f, 84.0 * P + 36.0 * C),
-        "assign_lists": (tm["assign_ms"] / ns, 12.0 * C + 16.0 * n),
-        "sweep_flow": (tm["sweep_ms"] / ns, tm["sweep_bytes"] / ns),
+        "assign_flow": (tm["assign_ms"] / ns, 12.0 * C + 16.0 * n),
+        "sweep_flow" if w.joints else "sweep_first": (tm["sweep_ms"] / ns, tm["sweep_bytes"] / ns),
     }
 
 

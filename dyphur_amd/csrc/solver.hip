@@ -1808,6 +1808,7 @@ struct dy_xpbd_s {
     bool timing = false;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     bool ev_pending = false;
+    bool ends_early = false;  // the timed sweep ends after iteration 0 when no contact is live
     dy_solver_timing acc{};
 };
 
@@ -1848,8 +1849,10 @@ int collect_timing(dy_xpbd_s *x) {
     x->acc.sweep_ms += b;
     // Algorithmic bytes of the sweep: per contact per iteration 36 B record
     // + 8 B lambda, per dynamic endpoint 80 B read + 52 B written, plus the
-    // per-iteration renormalisation (32 B per body).
-    x->acc.sweep_bytes += static_cast<double>(x->n_iters) *
+    // per-iteration renormalisation (32 B per body).  A contact-only dataflow
+    // sweep ends after its first iteration when no contact is left live.
+    const int ran = x->ends_early && !x->h_meta[kMLive] && x->n_iters > 1 ? 1 : x->n_iters;
+    x->acc.sweep_bytes += static_cast<double>(ran) *
                           (44.0 * x->stats.n_constraints + 132.0 * x->stats.dyn_endpoints + 32.0 * x->last_nb);
     x->ev_pending = false;
     return DY_OK;
@@ -2378,6 +2381,7 @@ int dy_xpbd_solve(dy_xpbd_t x, dy_stream_t s, const dy_contact_view *cv, const d
     if (x->timing) {
         DY_TRY(hipEventRecord(x->ev[3], st));
         x->ev_pending = true;
+        x->ends_early = swept && flow && !J;
     }
     scatter_bodies<<<ceil_div(nb, 256), 256, 0, st>>>(*bv, x->dyn.p, iters, words ? x->bw.p : nullptr, x->meta);
     DY_LAUNCH_CHECK();

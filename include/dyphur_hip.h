@@ -137,7 +137,7 @@ typedef struct dy_solver_timing {
     uint32_t solves;          /* solves timed */
     double assign_ms;         /* total class-assignment kernel time */
     double sweep_ms;          /* total sweep kernel time */
-    double sweep_bytes;       /* total algorithmic bytes of the timed sweeps */
+    double sweep_bytes;       /* total algorithmic bytes of the timed sweeps' iterations (those that ran) */
 } dy_solver_timing;
 
 /* Kernel timing of the broadphase, accumulated over builds while enabled: HIP

@@ -333,3 +333,21 @@ def test_later_iterations_by_words(gpu, monkeypatch, n, iters):
     assert np.max(np.abs(first["rot_w"] - once["rot_w"])) > 1e-4
     monkeypatch.setenv("DYPHUR_SWEEP_PAIR", "0")
     assert _same_bits(_solved(gpu, sc, a, b, fields, iters, 2), got)
+
+
+def test_timing_charges_the_iterations_that_ran(gpu):
+    """Ten iterations of which nine have nothing to do count as one, and all
+    count where contacts stay live."""
+    for sc, a, b, fields, iters, ran in [
+            (lambda c: (c[3], c[0], c[1], [np.zeros(900, np.float32)] * 7))(_contacts(300, 900)) + (10, 1),
+            _plates(60) + (4, 4)]:
+        print(f"[sweep bytes] nc={len(a)} iters={iters}", flush=True)
+        s = gpu.Stream()
+        db = gpu.DeviceBodies(sc, s)
+        solver = gpu.XpbdSolver(s, iters, len(a), 0.5)
+        cv, _keep = _view(gpu, s, np.asarray(a, np.uint32), np.asarray(b, np.uint32), fields)
+        solver.set_timing(True)
+        solver.solve(s, cv, db, sc.dt)
+        tm, st = solver.timing(s), solver.stats()
+        once = 44.0 * st["n_constraints"] + 132.0 * st["dyn_endpoints"] + 32.0 * sc.n
+        assert tm["solves"] == 1 and tm["sweep_bytes"] == ran * once
