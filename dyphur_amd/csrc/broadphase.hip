@@ -381,8 +381,9 @@ __global__ __launch_bounds__(kSgThreads) void morton_sort_grid(dy_body_view bv, 
 // square of the tiles.  Against the one-workgroup and one-XCD radix sorts (their
 // barriers and ballots on a few CUs): 64 bodies 18 -> 6 us, 1 025 23 -> 13,
 // 5 000 30 -> 14, 32 768 54 -> 19, 98 305 122 -> 41 (of it rank_merge 2.5, 3, 6
-// and 22); larger scenes keep the radix sort.  A key's count is of at most 8
-// tiles (kRankMax / kRankTile / kRankGroups), 16 bits.
+// and 22), 180 000 165 -> 90, 262 144 244 -> 156; larger scenes keep the radix
+// sort.  The line is where the counts end: a key's count is of at most 8 tiles
+// (kRankMax / kRankTile / kRankGroups), 16 bits.
 constexpr uint32_t kRankTile = 1024, kRankRows = 64, kRankGroups = 32, kRankMax = 262144;
 constexpr uint32_t kRankPad = 1u << 30;  // codes have 30 bits
 
